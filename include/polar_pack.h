@@ -366,6 +366,29 @@ int pp_quad_plug_codes(const uint32_t* codes, int64_t n_codes, const uint32_t* p
 int pp_plug_search(const uint32_t* plug_idx, int64_t plug_n, int64_t pos0, int64_t pld, int64_t rows,
                    int64_t slices, int64_t cols, int64_t* row_plug, void* stream);
 
+/*
+ * The quad layer packer (pack_quad_layer, quad_kernels.py:16-50) over n tuples of four
+ * equally laid out weight arrays w[m] (PP_F16 or PP_F32, aligned to 4 elements), on one stream:
+ *   pp_quad_pack_squares  for each model, sq[i] = w[i]^2 in float32 (sq 16-byte aligned, its
+ *                         length n rounded up to 4), whose mean the caller takes; clears meta[4]
+ *   pp_quad_pack_norm     meta[0..3] = sqrt(*means[m]), meta[4] = the largest norm of the
+ *                         tuples (w[m][i] / meta[m]) (NaN if any is)
+ *   pp_quad_pack_codes    codes[i] = the word [nq|q1|q2|q3] of tuple i, r_max = meta[4]*1.001
+ * The arithmetic is float32, operation by operation that of the reference's expressions.
+ */
+int pp_quad_pack_squares(const void* w, int dtype, int64_t n, float* sq, float* meta, void* stream);
+int pp_quad_pack_norm(const void* const* w, int dtype, int64_t n, const float* const* means, float* meta,
+                      void* stream);
+int pp_quad_pack_codes(const void* const* w, int dtype, int64_t n, double mu, double log_mu, const float* meta,
+                       uint32_t* codes, void* stream);
+
+/*
+ * bytes (a multiple of 4) of host memory to the device in the launch's own arguments: the
+ * host memory is read before the call returns and nothing waits for earlier work.  For
+ * tables of a few KB.  No counterpart in the reference.
+ */
+int pp_upload(void* dst, const void* src, int64_t bytes, void* stream);
+
 /* ------------------------------------------------------------------------ */
 /* Dual pack: 16-bit [amp 6 | phase 10] -> 2 models.                          */
 /* ------------------------------------------------------------------------ */
@@ -586,6 +609,17 @@ int pp_dual_stream(const pp_dual_proj* projs, int64_t n_projs,
                    const uint32_t* plug_idx, const void* plug_amp, const uint32_t* plug_ent, int64_t plug_n,
                    int64_t n_codes, const void* const* tails, const int64_t* tail_len,
                    int64_t M, void* stream);
+
+/*
+ * The dual layer packer (quantize_polar_bitpacked, polar_kernels.py:118-151) over n pairs of
+ * two contiguous weight arrays (PP_F16 or PP_F32, aligned to 4 elements): codes[i] =
+ * ((amp << 10) | phase) - 32768 and the fp16 maximum amplitude of each run of group_size
+ * pairs (a power of two in 8..512; 1 where it is not above 1e-10).  levels = 2^amp_bits - 1
+ * <= 63, num_phases <= 1024, log_mu = ln(1 + mu).  Every intermediate is rounded to the
+ * weights' type, as the reference's tensor expressions are.
+ */
+int pp_dual_pack(const void* w1, const void* w2, int dtype, int64_t n, int64_t group_size, int64_t num_phases,
+                 int levels, double mu, double log_mu, int16_t* codes, void* bmax, void* stream);
 
 /*
  * Group scales of a dual stream regrouped for pp_dual_stream's scale_tab (built once per

@@ -23,6 +23,7 @@ PP_ITEM_FP16 = 2
 vp = C.c_void_p
 i64 = C.c_int64
 i32 = C.c_int
+f64 = C.c_double
 
 
 class QuadProj(C.Structure):
@@ -112,6 +113,11 @@ EXPORTS = {
                                   vp, vp, i64, i64, vp]),
     "pp_dual_dequant_f16_t": (i32, [vp, i32, i64, vp, i64, vp, i32, vp, vp, i32, i32, vp, vp, i64, i64, vp, vp,
                                     i64, i64, vp]),
+    "pp_quad_pack_squares": (i32, [vp, i32, i64, vp, vp, vp]),
+    "pp_quad_pack_norm": (i32, [vp, i32, i64, vp, vp, vp]),
+    "pp_quad_pack_codes": (i32, [vp, i32, i64, f64, f64, vp, vp, vp]),
+    "pp_dual_pack": (i32, [vp, vp, i32, i64, i64, i64, i32, f64, f64, vp, vp, vp]),
+    "pp_upload": (i32, [vp, vp, i64, vp]),
 }
 
 _lock = threading.Lock()
@@ -167,6 +173,38 @@ def raw_stream(dev) -> int:
     import torch
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
     return torch._C._cuda_getCurrentRawStream(idx)
+
+
+def packable(ws) -> bool:
+    """Whether the packers' kernels may read these weights straight from memory: plain fp16 or
+    float32 device tensors of one type, shape and stride order, dense and 16-byte aligned, with
+    no transform in force (tracing, vmap, forward-mode, autocast or a dispatch mode) that has to
+    see the tensor expressions themselves."""
+    import torch
+    w0 = ws[0]
+    if w0.device.type != "cuda" or w0.dtype not in (torch.float16, torch.float32) \
+            or torch.get_default_device().type != "cpu":
+        return False
+    n = w0.numel()
+    if not 0 < n < 2 ** 31 or not (w0.is_contiguous() or (w0.dim() == 2 and w0.t().is_contiguous())):
+        return False
+    for w in ws:
+        if type(w) not in (torch.Tensor, torch.nn.Parameter) or torch._C._functorch.is_functorch_wrapped_tensor(w) \
+                or w.device != w0.device or w.dtype != w0.dtype or w.shape != w0.shape or w.stride() != w0.stride() \
+                or w.is_neg() or w.data_ptr() % 16:
+            return False
+    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_autocast_enabled("cuda")
+                or torch._C._len_torch_dispatch_stack() or torch.autograd.forward_ad._current_level >= 0)
+
+
+def upload(host, dev):
+    """A device copy of a small contiguous host tensor (a multiple of 4 bytes), carried in the
+    launches' arguments (pp_upload): unlike ``host.to(dev)`` it does not wait for queued work."""
+    import torch
+    out = torch.empty(host.shape, dtype=host.dtype, device=dev)
+    check(lib().pp_upload(out.data_ptr(), host.data_ptr(), host.numel() * host.element_size(), raw_stream(dev)),
+          "pp_upload")
+    return out
 
 
 def plug_search(idx, n: int, pos0: int, pld: int, rows: int, slices: int, cols: int, dev):

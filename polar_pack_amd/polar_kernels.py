@@ -24,6 +24,7 @@ torch.matmul).
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import torch
@@ -48,6 +49,10 @@ def quantize_polar_bitpacked(w1, w2, amp_bits=6, num_phases=1024, mu=255, group_
     cos_lut fp16[num_phases], sin_lut fp16[num_phases])`` on w1's device.
     """
     K, N = w1.shape
+    levels = (1 << amp_bits) - 1
+    log_mu = math.log(1 + mu)
+    if _pack_on_device(w1, w2, amp_bits, num_phases, mu, group_size):
+        return _pack_dual_device(w1, w2, levels, num_phases, mu, log_mu, group_size)
     amplitude = torch.sqrt(w1 ** 2 + w2 ** 2)
     phase = torch.atan2(w2, w1)
     phase_q = (torch.round((phase + math.pi) / (2 * math.pi) * num_phases).long() % num_phases).to(torch.int16)
@@ -60,17 +65,54 @@ def quantize_polar_bitpacked(w1, w2, amp_bits=6, num_phases=1024, mu=255, group_
     bmax = grouped.abs().max(dim=1, keepdim=True).values
     bmax = torch.where(bmax > 1e-10, bmax, torch.ones_like(bmax))
     norm = grouped / bmax
-    log_mu = math.log(1 + mu)
     compressed = torch.sign(norm) * torch.log1p(mu * norm.abs()) / log_mu
-    levels = (1 << amp_bits) - 1
     amp_q = torch.round(compressed * levels).clamp(0, levels).to(torch.int8).flatten()[:total].reshape(K, N)
     bmax = bmax.flatten().to(torch.float16)
     packed = pack_amp_phase(amp_q, phase_q)
+    amp_lut, cos_lut, sin_lut = (t.to(w1.device) for t in _layer_luts(levels, num_phases, mu, log_mu))
+    return packed, bmax, amp_lut, cos_lut, sin_lut
+
+
+def _layer_luts(levels, num_phases, mu, log_mu):
+    """(amp_lut, cos_lut, sin_lut) of a packed layer as fp16 host tensors (polar_kernels.py:142-150);
+    they depend on nothing but the code's parameters."""
     phases = torch.linspace(-math.pi, math.pi, num_phases + 1)[:-1]
-    cos_lut = torch.cos(phases).to(torch.float16).to(w1.device)
-    sin_lut = torch.sin(phases).to(torch.float16).to(w1.device)
     i = torch.arange(levels + 1, dtype=torch.float32)
-    amp_lut = ((torch.exp(i / levels * log_mu) - 1.0) / mu).to(torch.float16).to(w1.device)
+    return (((torch.exp(i / levels * log_mu) - 1.0) / mu).to(torch.float16), torch.cos(phases).to(torch.float16),
+            torch.sin(phases).to(torch.float16))
+
+
+@functools.lru_cache(maxsize=8)
+def _lut_block(levels, num_phases, mu, log_mu, default_dtype):
+    """[cos | sin | amp] of :func:`_layer_luts` as one host tensor (linspace follows torch's
+    default dtype, hence the key)."""
+    amp, cos, sin = _layer_luts(levels, num_phases, mu, log_mu)
+    return torch.cat([cos, sin, amp])
+
+
+def _pack_on_device(w1, w2, amp_bits, num_phases, mu, group_size):
+    """Whether pack.hip's one-pass packer takes the call: weights it can read (row-major: groups
+    run over the flattened layer), no gradient through the scales, codes that fit their fields and
+    groups of whole lanes (8 pairs) inside a wavefront."""
+    return (type(mu) in (int, float) and mu > 0 and type(amp_bits) is int and 1 <= amp_bits <= 6
+            and type(num_phases) is int and num_phases % 8 == 0 and 8 <= num_phases <= 1024
+            and type(group_size) is int and group_size in (8, 16, 32, 64, 128, 256, 512)
+            and nat.packable((w1, w2)) and w1.is_contiguous()
+            and not (torch.is_grad_enabled() and (w1.requires_grad or w2.requires_grad)))
+
+
+def _pack_dual_device(w1, w2, levels, num_phases, mu, log_mu, group_size):
+    """quantize_polar_bitpacked in one pass over the weights (pack.hip), the same codes, scales and LUTs."""
+    dev, n = w1.device, w1.numel()
+    with torch.cuda.device(dev):
+        packed = torch.empty(w1.shape, dtype=torch.int16, device=dev)
+        bmax = torch.empty(-(-n // group_size), dtype=torch.float16, device=dev)
+        nat.check(nat.lib().pp_dual_pack(w1.data_ptr(), w2.data_ptr(),
+                                         nat.PP_F16 if w1.dtype == torch.float16 else nat.PP_F32, n, group_size,
+                                         num_phases, levels, mu, log_mu, packed.data_ptr(), bmax.data_ptr(),
+                                         nat.raw_stream(dev)), "pp_dual_pack")
+        cos_lut, sin_lut, amp_lut = nat.upload(_lut_block(levels, num_phases, mu, log_mu, torch.get_default_dtype()),
+                                               dev).split([num_phases, num_phases, levels + 1])
     return packed, bmax, amp_lut, cos_lut, sin_lut
 
 

@@ -26,6 +26,7 @@ from __future__ import annotations
 
 import collections
 import ctypes
+import functools
 import math
 import threading
 import weakref
@@ -53,6 +54,8 @@ def pack_quad_layer(w1, w2, w3, w4, mu=MU):
     sin2, cos3, sin3] fp16[256] on w1.device, scales [4 floats])``.
     """
     ws = [w1, w2, w3, w4]
+    if type(mu) in (int, float) and nat.packable(ws):
+        return _pack_quad_device(ws, mu)
     s = [torch.sqrt((w.float() ** 2).mean()) for w in ws]
     wn = [w.float() / sk for w, sk in zip(ws, s)]
     r = torch.sqrt(wn[0] ** 2 + wn[1] ** 2 + wn[2] ** 2 + wn[3] ** 2)
@@ -66,14 +69,63 @@ def pack_quad_layer(w1, w2, w3, w4, mu=MU):
     q2 = torch.round(t2 / math.pi * 255).clip(0, 255)
     q3 = torch.round(t3 / (2 * math.pi) * 255).clip(0, 255)
     codes = _u32_words(nq, q1, q2, q3)
+    growth, angles = _lut_tables(mu)
+    luts = [t.to(w1.device) for t in ((growth * r_max / mu).to(torch.float16), *angles)]
+    return codes, luts, [float(sk) for sk in s]
+
+
+def _lut_tables(mu):
+    """What a layer's LUTs hold whatever its weights: exp(i/255 ln(1+mu)) - 1 in float32, which
+    r_max / mu scales to the norms, and the six fp16 angle tables (quad_kernels.py:39-49)."""
     i = torch.arange(256, dtype=torch.float32)
     half_turn = i / 255 * math.pi
     full_turn = i / 255 * 2 * math.pi
-    tables = [(torch.exp(i / 255 * log_mu) - 1) * r_max / mu,
-              torch.cos(half_turn), torch.sin(half_turn), torch.cos(half_turn), torch.sin(half_turn),
+    angles = [torch.cos(half_turn), torch.sin(half_turn), torch.cos(half_turn), torch.sin(half_turn),
               torch.cos(full_turn), torch.sin(full_turn)]
-    luts = [t.to(torch.float16).to(w1.device) for t in tables]
-    return codes, luts, [float(sk) for sk in s]
+    return torch.exp(i / 255 * math.log1p(mu)) - 1, [t.to(torch.float16) for t in angles]
+
+
+@functools.lru_cache(maxsize=8)
+def _lut_rows(mu):
+    """:func:`_lut_tables` as host tensors: the growth, and 7 fp16 rows whose first is the norms'."""
+    growth, angles = _lut_tables(mu)
+    return growth, torch.stack([torch.zeros_like(angles[0]), *angles])
+
+
+def _pack_quad_device(ws, mu):
+    """The packer's passes on the device (pack.hip), the same codes, LUTs and scales.  The means
+    stay torch's, whose summation order decides the scales' last bits.  The host waits once, for
+    the scales and the largest norm, while the codes are being written."""
+    w0, L = ws[0], nat.lib()
+    dev, n = w0.device, w0.numel()
+    dtype = nat.PP_F16 if w0.dtype == torch.float16 else nat.PP_F32
+    ptrs = nat.ptr_array([w.data_ptr() for w in ws])
+    log_mu = math.log1p(mu)
+    with torch.cuda.device(dev), torch.no_grad():
+        stream = nat.raw_stream(dev)
+        codes = torch.empty_like(w0, dtype=torch.int32)
+        sq = torch.empty(-(-n // 4) * 4, dtype=torch.float32, device=dev)
+        meta = torch.empty(5, dtype=torch.float32, device=dev)
+        host = torch.empty(5, dtype=torch.float32, pin_memory=True)
+        means = []
+        for p in ptrs:
+            nat.check(L.pp_quad_pack_squares(p, dtype, n, sq.data_ptr(), meta.data_ptr(), stream),
+                      "pp_quad_pack_squares")
+            means.append(sq[:n].mean())
+        nat.check(L.pp_quad_pack_norm(ptrs, dtype, n, nat.ptr_array([t.data_ptr() for t in means]), meta.data_ptr(),
+                                      stream), "pp_quad_pack_norm")
+        host.copy_(meta, non_blocking=True)
+        known = torch.cuda.Event()
+        known.record()
+        nat.check(L.pp_quad_pack_codes(ptrs, dtype, n, mu, log_mu, meta.data_ptr(), codes.data_ptr(), stream),
+                  "pp_quad_pack_codes")
+        known.synchronize()
+        *scales, top = host.tolist()
+        growth, rows = _lut_rows(mu)
+        rows = rows.clone()
+        rows[0] = growth * (top * 1.001) / mu
+        luts = nat.upload(rows, dev)
+    return codes.view(torch.uint32), list(luts.unbind(0)), scales
 
 
 def _lut_args(luts):
