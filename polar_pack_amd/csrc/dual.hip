@@ -20,32 +20,11 @@
 #include "dequant_t.h"
 #include "dual_kn.h"
 #include "dual_lds.h"
+#include "rows_common.h"
 
 #include <algorithm>
 
 namespace pp {
-
-constexpr int DREPL_A = 32;   // amplitude table replicas (b32 reads)
-constexpr int DREPL_C = 16;   // (cos, sin) table replicas (b64 reads)
-constexpr int DSEG = 512;     // codes per wave per row per step (64 lanes x 8)
-constexpr int rows_threads_dual(int MT) { return MT >= 4 ? 512 : 1024; }
-
-struct DualLds {
-  float amp[64 * DREPL_A];
-  float2 cs[1024 * DREPL_C];
-};
-
-__device__ __forceinline__ void dual_build_lds(DualLds& T, const DualLuts& L) {
-  for (int i = threadIdx.x; i < 64 * DREPL_A; i += blockDim.x) {
-    const int e = i / DREPL_A;
-    T.amp[i] = e < L.amp_n ? lut_at(L.amp, L.dtype, e) : 0.f;
-  }
-  for (int i = threadIdx.x; i < 1024 * DREPL_C; i += blockDim.x) {
-    const int e = i / DREPL_C;
-    T.cs[i] = e < L.phase_n ? make_float2(lut_at(L.cs[0], L.dtype, e), lut_at(L.cs[1], L.dtype, e))
-                            : make_float2(0.f, 0.f);
-  }
-}
 
 // 16-bit word as stored -> code (amp << 10 | phase)
 template <int LAYOUT>
@@ -64,204 +43,319 @@ struct DualGroup {
   }
 };
 
+// Batch 1..4 decode over the .dualpack stream layout.  A task is RG rows x one of `parts`
+// runs of 512-pair chunks of K; a task's parts are neighbouring waves of one workgroup, whose
+// sums meet in LDS, so the launch needs no workspace and no atomics.
+//
+// What bounds it: a Linear of a few million pairs is read in less time than a launch, a table
+// build and a reduction take, so the kernel is shaped around one round trip: the first chunk
+// and the task's place in the plug table (a 64-way search by the whole wave: three dependent
+// loads for 262,144 entries, in place of a search kernel of its own) travel while the tables
+// are built, and the host picks the parts that leave the fewest chunk times (dual_rows_plan).
+// Measured with 1 % plug entries, per call in a graph, against one to four rows a task without
+// look-ahead and a search kernel before it: 1531 x 4104 at 3 tokens 24.7 -> 11.9 us, 11008 x
+// 2048 at 1 / 2 tokens 30.4 / 36.9 -> 23.4 / 25.7, 2048 x 11016 at 2 tokens 99.7 -> 23.0, 256 x
+// 264 at 2 tokens 11.0 -> 6.5.  The large ones are bound by the decode's instructions (~12 a
+// pair and token) and table reads at two wavefronts a SIMD.
+constexpr int DR_NT = 512;       // threads per workgroup (one per CU: the tables take most of LDS)
+constexpr int DR_WAVES = DR_NT / 64;
+constexpr int DR_CHUNK = 512;    // pairs per wave, row and step: 8 per lane
+
 struct DualRowsArgs {
-  const void* codes;   // code of (row 0, k 0)
-  int64_t ldc;         // row stride (elements)
-  int64_t pos0;        // stream position of (row 0, 0)
+  const uint16_t* codes;   // code of (row 0, k 0)
+  int64_t ldc;             // row stride (elements)
+  int64_t pos0;            // stream position of (row 0, 0)
   const f16* x;
   int64_t x_sm;
   f16* out[2];
   int64_t o_sm, o_sn;
   int N, K, M;
-  int n_slices, slice_len;
-  int64_t n_tasks;
+  int tasks, parts, rounds;
   const f16* scales;
   DualGroup grp;
   DualLuts luts;
   const uint32_t* plug_idx;
   const f16* plug_amp;
-  const int64_t* rg_plug;
-  float* part;
-  int64_t part_stride;
-  uint32_t* counters;
+  int64_t plug_n;
 };
 
-template <int LAYOUT>
-__device__ __forceinline__ void dual_decode_one(const DualLds& T, uint32_t code, int ra, int rc, float& amp_n,
-                                                float2& cs) {
-  amp_n = T.amp[((code >> 10) & 63u) * DREPL_A + ra];
-  cs = T.cs[(code & 1023u) * DREPL_C + rc];
+// A wave's task.  Its pairs are addressed by o = their offset from row0's first pair + low,
+// low being that pair's place in its group: pair o is in group o / gs of `scales` up to the
+// next chunk boundary, where the groups restart.
+struct DrTask {
+  int row0, nrows, k0, k1;
+  rsrc_t codes;            // the rows from k0 (past the last row's k1 it reads 0)
+  const f16* scales;       // the first pair's group scale
+  uint32_t low;
+  uint32_t edge;           // o of the next chunk boundary, 0xFFFFFFFF if past the task's rows
+  uint32_t edge_group;     // its group
+};
+
+template <int RG>
+__device__ __forceinline__ DrTask dr_task(const DualRowsArgs& A, int t, int part) {
+  DrTask T;
+  const int chunks = (A.K + DR_CHUNK - 1) / DR_CHUNK;
+  T.row0 = min(t * RG, A.N);
+  T.nrows = t < A.tasks ? min(RG, A.N - T.row0) : 0;
+  T.k0 = (int)((int64_t)part * chunks / A.parts) * DR_CHUNK;
+  T.k1 = min(A.K, (int)((int64_t)(part + 1) * chunks / A.parts) * DR_CHUNK);
+  const bool any = T.nrows > 0 && T.k1 > T.k0;
+  T.codes = make_rsrc(A.codes + (int64_t)T.row0 * A.ldc + T.k0,
+                      any ? 2u * (uint32_t)((T.nrows - 1) * A.ldc + T.k1 - T.k0) : 0u);
+  const int64_t p = A.pos0 + (int64_t)T.row0 * A.ldc;
+  const int64_t c = p / A.grp.chunk, rem = p - c * A.grp.chunk, g = rem >> A.grp.log2gs;
+  T.scales = uniform_ptr(A.scales + c * A.grp.per_chunk + g);
+  T.low = (uint32_t)uniform((int)(rem & (A.grp.gs - 1)));
+  const int64_t edge = A.grp.chunk - (g << A.grp.log2gs);
+  const bool reaches = edge < (int64_t)T.low + RG * A.ldc;              // RG * ldc < 2^29
+  T.edge = (uint32_t)uniform(reaches ? (int)edge : -1);
+  T.edge_group = (uint32_t)uniform((int)(A.grp.per_chunk - g));
+  return T;
+}
+
+// Group of pair o.  Past the first boundary within the task a pair is d = o - edge pairs into
+// the following chunks; there are several only if a chunk is shorter than the task's rows.
+__device__ __forceinline__ uint32_t dr_group(const DualRowsArgs& A, const DrTask& T, uint32_t o) {
+  if (T.edge == 0xFFFFFFFFu) return o >> A.grp.log2gs;
+  if (o < T.edge) return o >> A.grp.log2gs;
+  uint32_t d = o - T.edge, g = T.edge_group;
+  if (d >= A.grp.chunk) {
+    const uint32_t q = d / (uint32_t)A.grp.chunk;
+    d -= q * (uint32_t)A.grp.chunk;
+    g += q * (uint32_t)A.grp.per_chunk;
+  }
+  return g + (d >> A.grp.log2gs);
+}
+
+template <int MT>
+struct DrX {
+  rsrc_t r[MT];
+};
+
+template <int MT, int RG>
+struct DrStep {
+  u32x4 q[RG];
+  f16 sc[RG];
+  u32x4 x[MT];
+};
+
+// A lane past the part's columns reads 0 for its pairs and activations, and the scale of the
+// part's last pairs (not used: dr_compute).
+template <int MT, int RG>
+__device__ __forceinline__ void dr_issue(const DualRowsArgs& A, const DrTask& T, const DrX<MT>& X, int k, int lane,
+                                         DrStep<MT, RG>& S) {
+  const int kk = k + 8 * lane, ld = (int)A.ldc;
+  const bool in = kk < T.k1;
+  const uint32_t voff = 2u * (uint32_t)(kk - T.k0);
+#pragma unroll
+  for (int r = 0; r < RG; ++r) vload128(S.q[r], in ? voff + 2u * (uint32_t)(r * ld) : OOB, T.codes);
+  const uint32_t o = T.low + (uint32_t)max(0, min(kk, T.k1 - 8));
+#pragma unroll
+  for (int r = 0; r < RG; ++r) {
+    const int row = max(0, min(r, T.nrows - 1));
+    S.sc[r] = T.scales[dr_group(A, T, o + (uint32_t)(row * ld))];
+  }
+#pragma unroll
+  for (int j = 0; j < MT; ++j) vload128c(S.x[j], in ? 2u * (uint32_t)kk : OOB, X.r[j]);
+}
+
+__device__ __forceinline__ f16 dr_x(const u32x4& x, int e) {
+  const uint32_t w = e < 2 ? x.x : e < 4 ? x.y : e < 6 ? x.z : x.w;
+  return __builtin_bit_cast(f16, (unsigned short)((e & 1) ? (w >> 16) : w));
+}
+
+// A lane's 8 pairs of a row share one group scale (8 | gs, 8 | chunk, 8 | positions), which
+// multiplies their partial sum once.  From 3 tokens on the amplitude goes into (cos, sin)
+// rather than into every token's activation.
+template <int MT, int RG, int LAYOUT>
+__device__ __forceinline__ void dr_compute(const char* lds, const DualLane& dl, const DrStep<MT, RG>& S, bool valid,
+                                           float (&acc)[RG][2][MT]) {
+#pragma unroll
+  for (int r = 0; r < RG; ++r) {
+    const uint32_t d4[4] = {S.q[r].x, S.q[r].y, S.q[r].z, S.q[r].w};
+    float l1[MT], l2[MT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) l1[j] = l2[j] = 0.f;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      float an[2];
+      float2 cs[2];
+      dual_lookup2<LAYOUT>(lds, d4[h], dl, an, cs);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const float wc = an[u] * cs[u].x, ws = an[u] * cs[u].y;
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+          const float x = (float)dr_x(S.x[j], 2 * h + u);
+          if constexpr (MT < 3) {
+            l1[j] = fmaf(an[u] * x, cs[u].x, l1[j]);
+            l2[j] = fmaf(an[u] * x, cs[u].y, l2[j]);
+          } else {
+            l1[j] = fmaf(x, wc, l1[j]);
+            l2[j] = fmaf(x, ws, l2[j]);
+          }
+        }
+      }
+    }
+    const float sc = valid ? (float)S.sc[r] : 0.f;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      acc[r][0][j] = fmaf(sc, l1[j], acc[r][0][j]);
+      acc[r][1][j] = fmaf(sc, l2[j], acc[r][1][j]);
+    }
+  }
+}
+
+// One window of 64 plug entries: entry e of the lane, if it lies in the task's rows, with what
+// its correction x * (plug - amp_lut * scale) * (cos, sin) needs.
+template <int MT>
+struct DrPlug {
+  int row;                 // row in the task, -1 for none
+  uint32_t code;
+  f16 sc, amp;
+  f16 x[MT];
+};
+
+template <int MT, int RG>
+__device__ __forceinline__ bool dr_plug_issue(const DualRowsArgs& A, const DrTask& T, int64_t e, uint32_t idx,
+                                              DrPlug<MT>& P) {
+  const int64_t pos = A.pos0 + (int64_t)T.row0 * A.ldc;
+  const int64_t off = e < A.plug_n ? (int64_t)idx - pos : -1;
+  const bool in = e < A.plug_n && off < (int64_t)T.nrows * A.ldc;       // ascending: the window ends past the rows
+  P.row = -1;
+  if (in && off >= 0) {
+    int row = 0;
+#pragma unroll
+    for (int r = 1; r < RG; ++r) row += off >= (int64_t)r * A.ldc ? 1 : 0;
+    const int64_t k = off - (int64_t)row * A.ldc;
+    if (k < A.K) {
+      P.row = row;
+      P.code = A.codes[(int64_t)(T.row0 + row) * A.ldc + k];
+      P.sc = T.scales[dr_group(A, T, T.low + (uint32_t)off)];
+      P.amp = A.plug_amp[e];
+#pragma unroll
+      for (int j = 0; j < MT; ++j) P.x[j] = j < A.M ? A.x[(int64_t)j * A.x_sm + k] : (f16)0.f;
+    }
+  }
+  return __ballot(in) != 0;
 }
 
 template <int MT, int RG, int LAYOUT>
-__global__ __launch_bounds__(rows_threads_dual(MT)) void dual_rows_kernel(const DualRowsArgs A) {
-  __shared__ DualLds T;
-  dual_build_lds(T, A.luts);
-  __syncthreads();
-  constexpr int WAVES = rows_threads_dual(MT) / 64;
-  constexpr int NV = RG * 2 * MT;
-  const int lane = threadIdx.x & 63;
-  const int ra = lane % DREPL_A, rc = lane % DREPL_C;
-  const int64_t gw = (int64_t)blockIdx.x * WAVES + (threadIdx.x >> 6);
-  const int64_t nw = (int64_t)gridDim.x * WAVES;
-  const int64_t t_begin = gw * A.n_tasks / nw, t_end = (gw + 1) * A.n_tasks / nw;
-  const uint16_t* codes16 = reinterpret_cast<const uint16_t*>(A.codes);
-  for (int64_t ti = t_begin; ti < t_end; ++ti) {
-    const int rg = (int)(ti / A.n_slices), slice = (int)(ti % A.n_slices);
-    const int row0 = rg * RG;
-    const int nrows = min(RG, A.N - row0);
-    const int k0 = slice * A.slice_len, k1 = min(A.K, k0 + A.slice_len);
-    const int len = k1 - k0;
-    const int64_t pos_row0 = A.pos0 + (int64_t)row0 * A.ldc;
+__device__ __forceinline__ void dr_plug_apply(const char* lds, const DualLane& dl, const DrPlug<MT>& P,
+                                              float (&acc)[RG][2][MT]) {
+  if (P.row < 0) return;
+  float an;
+  float2 cs;
+  dual_lookup1(lds, dual_half<LAYOUT>(P.code), dl, an, cs);
+  const float d = (float)P.amp - an * (float)P.sc;
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    const float xd = (float)P.x[j] * d;
+#pragma unroll
+    for (int r = 0; r < RG; ++r) {
+      acc[r][0][j] = r == P.row ? fmaf(xd, cs.x, acc[r][0][j]) : acc[r][0][j];
+      acc[r][1][j] = r == P.row ? fmaf(xd, cs.y, acc[r][1][j]) : acc[r][1][j];
+    }
+  }
+}
+
+template <int MT, int RG, int LAYOUT>
+__global__ __launch_bounds__(DR_NT) void dual_rows_kernel(const DualRowsArgs A) {
+  constexpr int MP = MT == 3 ? 4 : MT;              // the reduction takes a power of two
+  constexpr int NV = RG * 2 * MP, LNV = Log2<NV>::v;
+  __shared__ __attribute__((aligned(16))) char lds[DLDS_BYTES + 2 * DR_WAVES * NV * 4];
+  float* red = reinterpret_cast<float*>(lds + DLDS_BYTES);
+  const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
+  const int parts = uniform(A.parts), groups = DR_WAVES / parts;
+  const int part = wave % parts;
+  const DualLane dl = dual_lane(lane);
+  DrX<MT> X;
+#pragma unroll
+  for (int j = 0; j < MT; ++j) X.r[j] = make_rsrc(A.x + (int64_t)min(j, A.M - 1) * A.x_sm, j < A.M ? 2u * (uint32_t)A.K : 0u);
+  DrTask T;
+  DrStep<MT, RG> s0, s1;
+  int64_t e0 = 0;          // the lane's entry in the part's first window
+  uint32_t idx0 = 0;
+  auto task = [&](int round) {
+    T = dr_task<RG>(A, (int)blockIdx.x + (int)gridDim.x * (wave / parts + groups * round), part);
+    if (T.nrows > 0) dr_issue<MT, RG>(A, T, X, T.k0, lane, s0);
+  };
+  auto window = [&]() {
+    if (A.plug_n == 0 || T.nrows == 0) return;
+    e0 = wave_lower_bound(A.plug_idx, A.plug_n, A.pos0 + (int64_t)T.row0 * A.ldc, lane) + 64 * part + lane;
+    idx0 = A.plug_idx[min(e0, A.plug_n - 1)];
+  };
+  // the first chunk, then the LUTs, then the search: their round trips overlap
+  task(0);
+  if (A.luts.dtype == PP_F16) {
+    DualTables<DR_NT, LAYOUT, f16> tb;
+    tb.load(A.luts);
+    window();
+    tb.store(lds);
+  } else {
+    DualTables<DR_NT, LAYOUT, float> tb;
+    tb.load(A.luts);
+    window();
+    tb.store(lds);
+  }
+  for (int round = 0; round < A.rounds; ++round) {
+    if (round > 0) {
+      task(round);
+      window();
+    }
     float acc[RG][2][MT];
 #pragma unroll
     for (int r = 0; r < RG; ++r)
 #pragma unroll
       for (int j = 0; j < MT; ++j) acc[r][0][j] = acc[r][1][j] = 0.f;
-    const uint16_t* cb = codes16 + (int64_t)row0 * A.ldc + k0 + 8 * lane;
-    const f16* xb = A.x + k0 + 8 * lane;
-    // group of each row's first pair for this lane: (chunk index, offset in chunk), advanced
-    // by DSEG per step; 8 consecutive pairs never straddle a group (8 | gs, 8 | chunk, 8 | pos)
-    int64_t gc[RG], grem[RG];
-#pragma unroll
-    for (int r = 0; r < RG; ++r) {
-      const int64_t p = pos_row0 + (int64_t)r * A.ldc + k0 + 8 * lane;
-      gc[r] = p / A.grp.chunk;
-      grem[r] = p - gc[r] * A.grp.chunk;
-    }
-    for (int kb = 0; kb < len; kb += DSEG) {
-      const bool valid = kb + 8 * lane < len;
-      u32x4 q[RG];
-      float sc[RG];
-#pragma unroll
-      for (int r = 0; r < RG; ++r) {
-        if (r < nrows && valid) {
-          q[r] = load_nt(reinterpret_cast<const uint32_t*>(cb + (int64_t)r * A.ldc + kb));
-          sc[r] = (float)A.scales[gc[r] * A.grp.per_chunk + (grem[r] >> A.grp.log2gs)];
-        } else {
-          q[r] = u32x4{0u, 0u, 0u, 0u};
-          sc[r] = 0.f;
-        }
-        grem[r] += DSEG;
-        while (grem[r] >= A.grp.chunk) {
-          grem[r] -= A.grp.chunk;
-          ++gc[r];
-        }
+    if (T.nrows > 0) {
+      // the task's entries, 64 a window, the windows dealt over its parts
+      DrPlug<MT> P;
+      bool more = A.plug_n > 0 && dr_plug_issue<MT, RG>(A, T, e0, idx0, P);
+      for (int k = T.k0; k < T.k1; k += 2 * DR_CHUNK) {
+        dr_issue<MT, RG>(A, T, X, k + DR_CHUNK, lane, s1);
+        dr_compute<MT, RG, LAYOUT>(lds, dl, s0, k + 8 * lane < T.k1, acc);
+        if (k + DR_CHUNK >= T.k1) break;
+        dr_issue<MT, RG>(A, T, X, k + 2 * DR_CHUNK, lane, s0);
+        dr_compute<MT, RG, LAYOUT>(lds, dl, s1, k + DR_CHUNK + 8 * lane < T.k1, acc);
       }
-      float xv[MT][8];
-#pragma unroll
-      for (int j = 0; j < MT; ++j) {
-        if (valid && j < A.M) {
-          const f16x4 h0 = *reinterpret_cast<const f16x4*>(xb + (int64_t)j * A.x_sm + kb);
-          const f16x4 h1 = *reinterpret_cast<const f16x4*>(xb + (int64_t)j * A.x_sm + kb + 4);
-          xv[j][0] = (float)h0.x; xv[j][1] = (float)h0.y; xv[j][2] = (float)h0.z; xv[j][3] = (float)h0.w;
-          xv[j][4] = (float)h1.x; xv[j][5] = (float)h1.y; xv[j][6] = (float)h1.z; xv[j][7] = (float)h1.w;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) xv[j][e] = 0.f;
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < RG; ++r) {
-        const uint32_t d4[4] = {q[r].x, q[r].y, q[r].z, q[r].w};
-        float l1[MT], l2[MT];
-#pragma unroll
-        for (int j = 0; j < MT; ++j) l1[j] = l2[j] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint32_t code = dual_code<LAYOUT>((d4[e >> 1] >> ((e & 1) * 16)) & 0xFFFFu);
-          float an;
-          float2 cs;
-          dual_decode_one<LAYOUT>(T, code, ra, rc, an, cs);
-#pragma unroll
-          for (int j = 0; j < MT; ++j) {
-            const float xa = an * xv[j][e];
-            l1[j] = fmaf(xa, cs.x, l1[j]);
-            l2[j] = fmaf(xa, cs.y, l2[j]);
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < MT; ++j) {
-          acc[r][0][j] = fmaf(sc[r], l1[j], acc[r][0][j]);
-          acc[r][1][j] = fmaf(sc[r], l2[j], acc[r][1][j]);
-        }
+      for (int64_t e = e0; more;) {
+        dr_plug_apply<MT, RG, LAYOUT>(lds, dl, P, acc);
+        e += 64 * parts;
+        more = dr_plug_issue<MT, RG>(A, T, e, A.plug_idx[min(e, A.plug_n - 1)], P);
       }
     }
-    // plug: amplitude replaced by plug_amp at its position
-    if (A.rg_plug != nullptr) {
-      const int64_t plo = A.rg_plug[rg], phi = A.rg_plug[rg + 1];
-      for (int64_t p0 = plo; p0 < phi; p0 += 64) {
-        const int64_t p = p0 + lane;
-        if (p >= phi) continue;
-        const int64_t off = (int64_t)A.plug_idx[p] - pos_row0;
-        if (off < 0) continue;
-        const int64_t row = off / A.ldc;
-        const int k = (int)(off - row * A.ldc);
-        if (row >= nrows || k < k0 || k >= k1) continue;
-        const uint32_t code = dual_code<LAYOUT>(codes16[(int64_t)(row0 + row) * A.ldc + k]);
-        float an;
-        float2 cs;
-        dual_decode_one<LAYOUT>(T, code, ra, rc, an, cs);
-        const float sc = (float)A.scales[A.grp.of_pos(pos_row0 + row * A.ldc + k)];
-        const float d = (float)A.plug_amp[p] - an * sc;
-#pragma unroll
-        for (int j = 0; j < MT; ++j) {
-          if (j >= A.M) break;
-          const float xk = (float)A.x[(int64_t)j * A.x_sm + k];
-#pragma unroll
-          for (int r = 0; r < RG; ++r) {
-            if (r == row) {
-              acc[r][0][j] = fmaf(xk * d, cs.x, acc[r][0][j]);
-              acc[r][1][j] = fmaf(xk * d, cs.y, acc[r][1][j]);
-            }
-          }
-        }
-      }
-    }
-    float mine[2] = {0.f, 0.f};
+    float v[NV];
 #pragma unroll
     for (int r = 0; r < RG; ++r)
 #pragma unroll
       for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int j = 0; j < MT; ++j) {
-          const float v = wave_sum(acc[r][m][j]);
-          if (lane == r * MT + j) mine[m] = v;
-        }
-    // lane r*MT + j owns (row r, token j) of both models
-    const int r = lane / MT, j = lane % MT;
-    const bool owner = lane < RG * MT && r < nrows && j < A.M;
-    const int64_t off = (int64_t)j * A.o_sm + (int64_t)(row0 + r) * A.o_sn;
-    if (A.n_slices <= 1) {
-      if (owner) {
-        A.out[0][off] = (f16)mine[0];
-        A.out[1][off] = (f16)mine[1];
-      }
+        for (int j = 0; j < MP; ++j) v[(r * 2 + m) * MP + j] = j < MT ? acc[r][m][j] : 0.f;
+    float y = wave_transpose_reduce<LNV>(v, lane);
+    constexpr int LOW = 6 - LNV;
+    const bool owns = (lane & ((1 << LOW) - 1)) == 0;
+    const int i = lane >> LOW;
+    auto store = [&](int t, int vi, float val) {
+      const int r = vi / (2 * MP), m = vi / MP % 2, j = vi % MP, row = t * RG + r;
+      if (t < A.tasks && row < A.N && j < A.M)
+        (m == 0 ? A.out[0] : A.out[1])[(int64_t)j * A.o_sm + (int64_t)row * A.o_sn] = (f16)val;
+    };
+    if (parts == 1) {
+      if (owns) store((int)blockIdx.x + (int)gridDim.x * (wave + groups * round), i, y);
       continue;
     }
-    float* grp = A.part + (int64_t)rg * A.part_stride;
-    if (lane < RG * MT) {
-      grp[(int64_t)slice * NV + 2 * lane] = mine[0];
-      grp[(int64_t)slice * NV + 2 * lane + 1] = mine[1];
+    // two buffers in turn: a wave writes a buffer again only after the next round's barrier,
+    // which every reader of this round has passed
+    float* rb = red + (round & 1) * DR_WAVES * NV;
+    if (owns) rb[wave * NV + i] = y;
+    __syncthreads();
+    if ((int)threadIdx.x < groups * NV) {
+      const int g = threadIdx.x / NV, vi = threadIdx.x % NV;
+      float s = 0.f;
+      for (int p = 0; p < parts; ++p) s += rb[(g * parts + p) * NV + vi];
+      store((int)blockIdx.x + (int)gridDim.x * (g + groups * round), vi, s);
     }
-    __threadfence();
-    uint32_t prev = 0;
-    if (lane == 0) prev = atomicAdd(A.counters + rg, 1u);
-    prev = __shfl(prev, 0, 64);
-    if (prev != (uint32_t)(A.n_slices - 1)) continue;
-    __threadfence();
-    if (lane < RG * MT) {
-      float s0 = 0.f, s1 = 0.f;
-      for (int s = 0; s < A.n_slices; ++s) {
-        s0 += __builtin_nontemporal_load(grp + (int64_t)s * NV + 2 * lane);
-        s1 += __builtin_nontemporal_load(grp + (int64_t)s * NV + 2 * lane + 1);
-      }
-      if (owner) {
-        A.out[0][off] = (f16)s0;
-        A.out[1][off] = (f16)s1;
-      }
-    }
-    if (lane == 0) A.counters[rg] = 0u;
   }
 }
 
@@ -491,78 +585,60 @@ __global__ __launch_bounds__(256) void dual_ws_gemm_kernel(const DualWsGemmArgs 
   A.out[1][i * A.o_sm + n * A.o_sn] = (f16)a1;
 }
 
-__global__ void dual_zero_u32_kernel(uint32_t* p, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0u;
-}
-
-__global__ void dual_rowgroup_plug_kernel(const uint32_t* plug_idx, int64_t plug_n, int64_t pos0, int64_t ldc,
-                                          int rows_per_group, int n_rowgroups, int N, int64_t* rg_plug) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g > n_rowgroups) return;
-  const int64_t row = min<int64_t>((int64_t)g * rows_per_group, N);
-  const int64_t key = pos0 + row * ldc;
-  int64_t lo = 0, hi = plug_n;
-  while (lo < hi) {
-    const int64_t mid = (lo + hi) >> 1;
-    if ((int64_t)plug_idx[mid] < key) lo = mid + 1;
-    else hi = mid;
-  }
-  rg_plug[g] = lo;
-}
-
 // ------------------------------------------------------------------------------------------
 // host side
-static int dual_round_mt(int64_t M) { return M <= 1 ? 1 : M <= 2 ? 2 : 4; }
-static int dual_rows_rg(int mt) { return mt == 1 ? 4 : (mt == 2 ? 2 : 1); }
 
 static bool dual_fast_ok(const void* a, int64_t a_sm, int64_t a_sk, const void* codes, int64_t c_sk, int64_t c_sn,
                          int64_t elem_base, int64_t chunk, int64_t gs, int64_t M, int64_t K) {
   return c_sk == 1 && c_sn % 8 == 0 && c_sn >= K && K % 8 == 0 && K > 0 && aligned(codes, 16) && M >= 1 &&
          M <= 4 && chunk > 0 && chunk % 8 == 0 && gs >= 8 && (gs & (gs - 1)) == 0 && elem_base % 8 == 0 &&
-         (a_sk == 1 || K == 1) && (M == 1 || a_sm % 4 == 0) && aligned(a, 8);
+         (a_sk == 1 || K == 1) && (M == 1 || a_sm % 4 == 0) && aligned(a, 8) &&
+         c_sn < (1ll << 26);          // 32-bit offsets over a task's rows
 }
 
-struct DualPlan {
-  int rg, n_rowgroups, n_slices, slice_len;
-  int64_t n_tasks, part_bytes, counter_bytes, plug_bytes;
-  int64_t total() const { return part_bytes + counter_bytes + plug_bytes; }
+struct DualRowsPlan {
+  int rg, tasks, parts, rounds;
 };
 
-static DualPlan dual_plan(int64_t M, int64_t N, int64_t K, int64_t plug_n) {
-  DualPlan p;
-  const int mt = dual_round_mt(M);
-  p.rg = dual_rows_rg(mt);
-  p.n_rowgroups = (int)((N + p.rg - 1) / p.rg);
-  const int64_t waves = (int64_t)device_cu_count() * (rows_threads_dual(mt) / 64);
-  const int64_t segs = (K + DSEG - 1) / DSEG;
-  int64_t want = (4 * waves + p.n_rowgroups - 1) / p.n_rowgroups;
-  want = std::max<int64_t>(1, std::min<int64_t>(want, std::max<int64_t>(1, K / 4096)));
-  const int64_t sps = (segs + want - 1) / want;
-  p.slice_len = (int)(sps * DSEG);
-  p.n_slices = (int)((K + p.slice_len - 1) / p.slice_len);
-  p.n_tasks = (int64_t)p.n_rowgroups * p.n_slices;
-  const int nv = p.rg * 2 * mt;
-  p.part_bytes = p.n_slices > 1 ? ((int64_t)p.n_rowgroups * p.n_slices * nv * 4 + 255) / 256 * 256 : 0;
-  p.counter_bytes = p.n_slices > 1 ? ((int64_t)p.n_rowgroups * 4 + 255) / 256 * 256 : 0;
-  p.plug_bytes = plug_n > 0 ? ((int64_t)(p.n_rowgroups + 1) * 8 + 255) / 256 * 256 : 0;
-  return p;
+// Rows per task (8 or 4, from 3 tokens 4 or 2), parts of K per task (1, 2, 4 or 8 neighbouring
+// waves of a workgroup) and rounds of tasks.  Two costs decide, both in rows x chunks: what the
+// busiest workgroup decodes (its 8 waves share the CU's units) and what its slowest wave does
+// one after another, an item's reduction and stores counted as a chunk of 4 rows.
+static DualRowsPlan dual_rows_plan(int mt, int64_t N, int64_t K) {
+  const int64_t chunks = (K + DR_CHUNK - 1) / DR_CHUNK, cus = device_cu_count();
+  DualRowsPlan best = {};
+  int64_t least = INT64_MAX;
+  for (int rg = mt <= 2 ? 8 : 4; rg >= (mt <= 2 ? 4 : 2); rg /= 2) {
+    const int64_t tasks = (N + rg - 1) / rg;
+    for (int parts = 1; parts <= DR_WAVES && parts <= chunks; parts *= 2) {
+      const int64_t slots = cus * (DR_WAVES / parts), rounds = (tasks + slots - 1) / slots;
+      const int64_t wave = rounds * (rg * ((chunks + parts - 1) / parts) + 4);
+      const int64_t group = (tasks + cus - 1) / cus * (rg * chunks + 4 * parts);
+      const int64_t cost = wave + group / 4;
+      if (cost < least) {
+        least = cost;
+        best = {rg, (int)tasks, parts, (int)rounds};
+      }
+    }
+  }
+  return best;
 }
 
 template <int MT, int RG, int LAYOUT>
 static int launch_dual_rows(const DualRowsArgs& A, hipStream_t st) {
-  hipLaunchKernelGGL((dual_rows_kernel<MT, RG, LAYOUT>), dim3(device_cu_count()), dim3(rows_threads_dual(MT)), 0,
-                     st, A);
+  hipLaunchKernelGGL((dual_rows_kernel<MT, RG, LAYOUT>), dim3((unsigned)std::min(device_cu_count(), A.tasks)),
+                     dim3(DR_NT), 0, st, A);
   PP_LAUNCH_CHECK();
   return PP_OK;
 }
 
 template <int LAYOUT>
-static int dispatch_dual_rows(const DualRowsArgs& A, int mt, hipStream_t st) {
+static int dispatch_dual_rows(const DualRowsArgs& A, int mt, int rg, hipStream_t st) {
   switch (mt) {
-    case 1: return launch_dual_rows<1, 4, LAYOUT>(A, st);
-    case 2: return launch_dual_rows<2, 2, LAYOUT>(A, st);
-    default: return launch_dual_rows<4, 1, LAYOUT>(A, st);
+    case 1: return rg == 8 ? launch_dual_rows<1, 8, LAYOUT>(A, st) : launch_dual_rows<1, 4, LAYOUT>(A, st);
+    case 2: return rg == 8 ? launch_dual_rows<2, 8, LAYOUT>(A, st) : launch_dual_rows<2, 4, LAYOUT>(A, st);
+    case 3: return rg == 4 ? launch_dual_rows<3, 4, LAYOUT>(A, st) : launch_dual_rows<3, 2, LAYOUT>(A, st);
+    default: return rg == 4 ? launch_dual_rows<4, 4, LAYOUT>(A, st) : launch_dual_rows<4, 2, LAYOUT>(A, st);
   }
 }
 
@@ -603,7 +679,7 @@ extern "C" int64_t pp_dual_gemm_workspace_size(const void* a, int64_t a_sm, int6
                                                int64_t elem_base, int64_t plug_n, int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0) return 0;
   if (dual_fast_ok(a, a_sm, a_sk, codes, c_sk, c_sn, elem_base, chunk_size, group_size, M, K))
-    return dual_plan(M, N, K, plug_n).total();
+    return 0;
   // (K,N) codes: blocks of up to 8 tokens, one after another, sharing the workspace (the
   // last block may have 1..7 tokens: the larger of the 4- and 8-token needs covers it)
   if (dual_kn_ok(a, a_sm, a_sk, codes, c_sk, c_sn, group_size, chunk_size, std::min<int64_t>(M, 8), N, K))
@@ -781,12 +857,10 @@ extern "C" int pp_dual_gemm(const void* a, int64_t a_sm, int64_t a_sk, const voi
   PP_REQUIRE(N < (1ll << 31) && K < (1ll << 31), "N and K must be < 2^31");
   const DualLuts L = make_dual_luts(amp_lut, amp_lut_n, cos_lut, sin_lut, phase_n, lut_dtype);
   if (dual_fast_ok(a, a_sm, a_sk, codes, c_sk, c_sn, elem_base, chunk_size, group_size, M, K)) {
-    const DualPlan p = dual_plan(M, N, K, plug_n);
-    PP_REQUIRE(workspace_bytes >= p.total() && (p.total() == 0 || workspace != nullptr),
-               "workspace too small: need %lld bytes", (long long)p.total());
-    char* ws = reinterpret_cast<char*>(workspace);
+    const int mt = (int)M;
+    const DualRowsPlan p = dual_rows_plan(mt, N, K);
     DualRowsArgs A = {};
-    A.codes = codes;
+    A.codes = reinterpret_cast<const uint16_t*>(codes);
     A.ldc = c_sn;
     A.pos0 = elem_base;
     A.x = reinterpret_cast<const f16*>(a);
@@ -798,9 +872,9 @@ extern "C" int pp_dual_gemm(const void* a, int64_t a_sm, int64_t a_sk, const voi
     A.N = (int)N;
     A.K = (int)K;
     A.M = (int)M;
-    A.n_slices = p.n_slices;
-    A.slice_len = p.slice_len;
-    A.n_tasks = p.n_tasks;
+    A.tasks = p.tasks;
+    A.parts = p.parts;
+    A.rounds = p.rounds;
     A.scales = reinterpret_cast<const f16*>(bmax);
     A.grp.gs = group_size;
     A.grp.chunk = chunk_size;
@@ -810,24 +884,9 @@ extern "C" int pp_dual_gemm(const void* a, int64_t a_sm, int64_t a_sk, const voi
     A.luts = L;
     A.plug_idx = plug_idx;
     A.plug_amp = reinterpret_cast<const f16*>(plug_amp);
-    const int mt = dual_round_mt(M);
-    A.part = p.part_bytes ? reinterpret_cast<float*>(ws) : nullptr;
-    A.part_stride = (int64_t)p.n_slices * p.rg * 2 * mt;
-    A.counters = p.counter_bytes ? reinterpret_cast<uint32_t*>(ws + p.part_bytes) : nullptr;
-    if (p.counter_bytes) {
-      const int64_t nc = p.counter_bytes / 4;
-      hipLaunchKernelGGL(dual_zero_u32_kernel, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, st, A.counters, nc);
-      PP_LAUNCH_CHECK();
-    }
-    if (plug_n > 0) {
-      int64_t* rgp = reinterpret_cast<int64_t*>(ws + p.part_bytes + p.counter_bytes);
-      hipLaunchKernelGGL(dual_rowgroup_plug_kernel, dim3((p.n_rowgroups + 1 + 255) / 256), dim3(256), 0, st,
-                         plug_idx, plug_n, elem_base, c_sn, p.rg, p.n_rowgroups, (int)N, rgp);
-      PP_LAUNCH_CHECK();
-      A.rg_plug = rgp;
-    }
-    return code_layout == PP_DUAL_U16_BE ? dispatch_dual_rows<PP_DUAL_U16_BE>(A, mt, st)
-                                         : dispatch_dual_rows<PP_DUAL_I16_OFFSET>(A, mt, st);
+    A.plug_n = plug_n;
+    return code_layout == PP_DUAL_U16_BE ? dispatch_dual_rows<PP_DUAL_U16_BE>(A, mt, p.rg, st)
+                                         : dispatch_dual_rows<PP_DUAL_I16_OFFSET>(A, mt, p.rg, st);
   }
   if (dual_kn_ok(a, a_sm, a_sk, codes, c_sk, c_sn, group_size, chunk_size, std::min<int64_t>(M, 8), N, K)) {
     for (int64_t i0 = 0; i0 < M; i0 += 8) {

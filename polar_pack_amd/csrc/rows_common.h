@@ -117,6 +117,22 @@ struct Log2<1> {
   static constexpr int v = 0;
 };
 
+// The first j in [0, n) with idx[j] >= key (n if none), idx ascending, found by a whole
+// wavefront: each round its lanes probe 64 evenly spaced entries, so n entries take
+// ceil(log64(n)) dependent loads.  Every lane must take part; all get the result.
+__device__ __forceinline__ int64_t wave_lower_bound(const uint32_t* idx, int64_t n, int64_t key, int lane) {
+  int64_t lo = 0;
+  while (n > 0) {
+    const int64_t step = (n + 63) / 64, i = lane * step;
+    const bool below = i < n && (int64_t)idx[lo + i] < key;
+    const int c = __popcll(__ballot(below));        // lanes 0 .. c-1: the probes ascend
+    if (c == 0) return lo;
+    lo += (c - 1) * step + 1;                       // past the last entry known below
+    n = min(step, n - (c - 1) * step) - 1;          // up to the next probe, which is not
+  }
+  return lo;
+}
+
 // A wavefront's segment range [seg_bounds[gw], seg_bounds[gw + 1]) (seg_bounds holds
 // n_waves + 1 entries).  issue() starts vector loads, so the round trip runs under the
 // LDS table build instead of before it (a scalar load there would be waited for by the
