@@ -367,6 +367,28 @@ int pp_plug_search(const uint32_t* plug_idx, int64_t plug_n, int64_t pos0, int64
                    int64_t slices, int64_t cols, int64_t* row_plug, void* stream);
 
 /*
+ * Fused decode of (K,N) codes (unit column stride, row stride ldk words) with fp16 tables for 1
+ * to 32 tokens, no plug table (quad_kernels.py:103-159): strips of columns x slices of K.
+ *   pp_quad_strip_ok              1 if it reads these operands: lut_dtype PP_F16, K % 8 == 0 (M > 1:
+ *                                 K % 32 == 0), N and ldk multiples of 4 words and codes 16-byte
+ *                                 aligned to 16 tokens (2 words, 8 bytes above), activations
+ *                                 16-byte aligned with a_sm % 8 == 0, K * ldk < 2^29
+ *   pp_quad_strip_workspace_size  bytes of workspace (the slices' float32 sums; any contents)
+ *   pp_quad_strip_counts          bytes of counts, zero on entry and left zero (one token in several
+ *                                 slices; launches that share them must not overlap)
+ * One token: float32 weights; more: weights rounded to fp16 for the matrix cores, float32 sums.
+ * Outputs (M,N), element (j, n) at out[m] + j*o_sm + n*o_sn.
+ */
+int pp_quad_strip_ok(const void* codes, int64_t ldk, const void* a, int64_t a_sm, int lut_dtype, int64_t M, int64_t N,
+                     int64_t K);
+int64_t pp_quad_strip_workspace_size(int64_t M, int64_t N, int64_t K);
+int64_t pp_quad_strip_counts(int64_t M, int64_t N, int64_t K);
+int pp_quad_strip(const uint32_t* codes, int64_t ldk, const void* a, int64_t a_sm, const void* const* luts,
+                  int lut_dtype, const float* scales, void* const* out, int64_t o_sm, int64_t o_sn, int64_t M,
+                  int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* counts, int64_t counts_bytes,
+                  void* stream);
+
+/*
  * The quad layer packer (pack_quad_layer, quad_kernels.py:16-50) over n tuples of four
  * equally laid out weight arrays w[m] (PP_F16 or PP_F32, aligned to 4 elements), on one stream:
  *   pp_quad_pack_squares  for each model, sq[i] = w[i]^2 in float32 (sq 16-byte aligned, its

@@ -305,6 +305,8 @@ def _quad_gemm(a, codes, lut_ptrs, lut_dtype, sc, pi, pv, pn, elem_base, outs, L
     N = codes.shape[1]
     if a.stride(1) != 1 or a.data_ptr() % 16 or (M > 1 and a.stride(0) % 8):
         a = a.contiguous()
+    if M == 1 and not pn and _quad_strip(a, codes, lut_ptrs, lut_dtype, sc, outs, L, dev):
+        return
     ws_bytes = L.pp_quad_gemm_workspace_size(a.data_ptr(), a.stride(0), a.stride(1), codes.data_ptr(),
                                              codes.stride(0), codes.stride(1), pn, M, N, K)
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
@@ -314,6 +316,30 @@ def _quad_gemm(a, codes, lut_ptrs, lut_dtype, sc, pi, pv, pn, elem_base, outs, L
                         nat.ptr_array([o.data_ptr() for o in outs]), outs[0].stride(0), outs[0].stride(1),
                         M, N, K, ws.data_ptr() if ws is not None else None, ws_bytes, stream)
     nat.check(rc, "pp_quad_gemm")
+
+
+def _quad_strip(a, codes, lut_ptrs, lut_dtype, sc, outs, L, dev):
+    """(K,N) codes at 1-32 tokens without plug entries: the strip kernels (pp_quad_strip), if they
+    read these operands (fp16 tables); False if not."""
+    M, K = a.shape
+    N = codes.shape[1]
+    if codes.stride(1) != 1:
+        return False
+    ldk, a_sm = codes.stride(0), a.stride(0)
+    if not L.pp_quad_strip_ok(codes.data_ptr(), ldk, a.data_ptr(), a_sm, lut_dtype, M, N, K):
+        return False
+    ws_bytes = L.pp_quad_strip_workspace_size(M, N, K)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+    n_counts = L.pp_quad_strip_counts(M, N, K)
+    counts, wkey = nat.zero_workspace(dev, n_counts)
+    rc = L.pp_quad_strip(codes.data_ptr(), ldk, a.data_ptr(), a_sm, lut_ptrs, lut_dtype, sc,
+                         nat.ptr_array([o.data_ptr() for o in outs]), outs[0].stride(0), outs[0].stride(1), M, N, K,
+                         ws.data_ptr() if ws is not None else None, ws_bytes,
+                         counts.data_ptr() if counts is not None else None, n_counts, nat.raw_stream(dev))
+    if rc:
+        nat.drop_workspace(wkey)
+    nat.check(rc, "pp_quad_strip")
+    return True
 
 
 def transposed_plug(idx, vals, elem_base, ldk, K, N):
@@ -359,6 +385,8 @@ def _quad_big(a, codes, layout, lut_ptrs, lut_dtype, sc, keep, pn, elem_base, ou
     N = codes.shape[1]
     if a.stride(1) != 1 or a.data_ptr() % 16 or (M > 1 and a.stride(0) % 8):
         a = a.contiguous()
+    if layout == nat.PP_QUAD_KN and M > 1 and not pn and _quad_strip(a, codes, lut_ptrs, lut_dtype, sc, outs, L, dev):
+        return outs
     plan = (ctypes.c_int64 * 2)()
     nat.check(L.pp_quad_big_plan(M, N, K, layout, ctypes.byref(plan, 0), ctypes.byref(plan, 8)), "pp_quad_big_plan")
     slices, cols = int(plan[0]), int(plan[1])

@@ -68,11 +68,11 @@ class Route:
 
 def kn_big_min_m(K: int, N: int, has_plug: bool) -> int:
     """(K,N) codes without plug entries: the fused matrix-core kernel from 2 tokens when N <= K,
-    from 3 when N > K; the (K,N) row kernel below (graph-replayed, row kernel against fused
-    kernel at 1 / 2 / 4 / 8 tokens: 4096x4096 23.3 / 29.6 / 36.6 / 45.5 against 27.6 / 27.4 /
-    27.4 / 27.4 us; K x N = 11008x2048 27.7 / 34.4 / 42.2 / 53.9 against 32.2 / 32.4 / 32.5 /
-    32.3; 2048x11008 25.6 / 33.9 / 41.9 / 56.3 against 38.4 / 38.4 / 40.6 / 40.7, 3 tokens 41.3
-    against 39.5)."""
+    from 3 when N > K; float32 weights below.  Graph-replayed, the (K,N) row kernel at 1 / 2 / 4
+    / 8 tokens: 4096x4096 23.3 / 29.6 / 36.6 / 45.5 us, K x N = 2048x11008 25.6 / 33.9 / 41.9 /
+    56.3; the fused kernel's strips (quad_strip.hip) at 2 / 16 tokens 21.3 / 23.4 and 24 / 26.4.
+    2 tokens stay float32 when N > K, where the row kernel once was the faster one, so that
+    those calls lose no precision."""
     return 2 if N <= K else 3
 
 

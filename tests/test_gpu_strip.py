@@ -1,0 +1,113 @@
+"""The strip kernels of (K,N) quad codes (pp_quad_strip, 1-32 tokens, fp16 tables) against float64
+products: partial strips and row units, one and several slices of K, more than one round of items,
+rows wider than the codes, tokens around a tile, tables whose q1 and q2 differ, and the counts left
+zero."""
+import numpy as np
+import pytest
+import torch
+
+from parity import assert_gemv_close, normwise
+from polar_pack_amd import _native as nat
+from polar_pack_amd import quad_kernels as qk
+from refs import kn_mfma_reference
+from test_gpu_big import fp16_luts, random_codes, u32
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+# K, N, row stride: below a strip, ragged, one slice of many rounds (20,000 columns), many slices
+SHAPES = [(32, 4, 4), (256, 36, 40), (96, 300, 520), (2080, 1000, 1000), (64, 20_000, 20_000), (8192, 256, 256)]
+
+
+def check(got, exact, what):
+    """Against the exact decode.  A weight's rounding to fp16 moves it by at most 2^-11 of itself, so
+    over random signs an output moves by a standard deviation of at most 2^-11 / sqrt(3) of the
+    outputs' root mean square (that of sqrt(K) random terms): held to 8 of them."""
+    for m in range(4):
+        g = got[m].float().cpu().numpy()
+        rms = np.sqrt((exact[m] ** 2).mean(axis=1, keepdims=True))       # ~ sqrt(K) x the rms term
+        assert_gemv_close(g, exact[m], f"{what} model {m}", bound=8 * 2.0 ** -11 / np.sqrt(3) * rms)
+        assert normwise(g, exact[m]) <= 1e-3, f"{what} model {m}"
+
+
+@pytest.mark.parametrize("K,N,ldk", SHAPES + [(40, 68, 68), (4104, 132, 136)])
+def test_one_token(K, N, ldk):
+    wide = random_codes((K, ldk), K + N)
+    luts, scales = fp16_luts(K + N, split=N % 8 == 0)
+    a = np.random.default_rng(N).standard_normal((1, K)).astype(np.float16)
+    view = u32(wide).to(DEV)[:, :N]
+    dl = [t.to(DEV) for t in luts]
+    assert nat.lib().pp_quad_strip_ok(view.data_ptr(), ldk, 0, K, nat.PP_F16, 1, N, K)
+    assert qk.quad_call_route(view, 1) == "kn"
+    exact = kn_mfma_reference(a, wide[:, :N], luts, scales)[0]
+    for rep in range(2):
+        got = qk.quad_bitpacked(torch.from_numpy(a).to(DEV), view, dl, scales)
+        torch.cuda.synchronize()
+        for m in range(4):                    # float32 weights: no fp16 rounding allowed for
+            assert_gemv_close(got[m].float().cpu().numpy(), exact[m], f"model {m} call {rep}", rtol=5.1e-4)
+
+
+@pytest.mark.parametrize("M", [2, 15, 16, 17, 32])
+@pytest.mark.parametrize("K,N,ldk", SHAPES)
+def test_matrix_core_tokens(K, N, ldk, M):
+    wide = random_codes((K, ldk), K + N + M)
+    luts, scales = fp16_luts(K + M, split=M % 2 == 0)
+    a = np.random.default_rng(N + M).standard_normal((M, K)).astype(np.float16)
+    view = u32(wide).to(DEV)[:, :N]
+    assert nat.lib().pp_quad_strip_ok(view.data_ptr(), ldk, 0, K, nat.PP_F16, M, N, K)
+    got = qk.quad_bitpacked(torch.from_numpy(a).to(DEV), view, [t.to(DEV) for t in luts], scales, fused=True)
+    check(got, kn_mfma_reference(a, wide[:, :N], luts, scales)[0], f"M={M}")
+
+
+@pytest.mark.parametrize("M", [1, 5, 20])
+def test_c_abi_workspace_and_strided_outputs(M):
+    """Any workspace contents, counts zero before and after, outputs with a column stride, and the
+    columns between left alone."""
+    K, N = 4096, 200
+    codes = random_codes((K, N), 9)
+    luts, scales = fp16_luts(9)
+    a = np.random.default_rng(M).standard_normal((M, K)).astype(np.float16)
+    L = nat.lib()
+    dc, da, dl = u32(codes).to(DEV), torch.from_numpy(a).to(DEV), [t.to(DEV) for t in luts]
+    ptrs, dt = qk._lut_args(dl)
+    n_ws, n_counts = L.pp_quad_strip_workspace_size(M, N, K), L.pp_quad_strip_counts(M, N, K)
+    assert n_ws > 0 and (n_counts > 0) == (M == 1)
+    ws = torch.full((n_ws // 4,), float("nan"), device=DEV)
+    counts = torch.zeros(max(n_counts // 4, 1), dtype=torch.int32, device=DEV)
+    wide = [torch.full((M, 2 * N), 7.0, dtype=torch.float16, device=DEV) for _ in range(4)]
+    ref = kn_mfma_reference(a, codes, luts, scales)[0]
+    for rep in range(2):
+        rc = L.pp_quad_strip(dc.data_ptr(), N, da.data_ptr(), K, ptrs, dt, nat.float_array(scales),
+                             nat.ptr_array([w.data_ptr() for w in wide]), 2 * N, 2, M, N, K, ws.data_ptr(), n_ws,
+                             counts.data_ptr(), n_counts, torch.cuda.current_stream(DEV).cuda_stream)
+        nat.check(rc, "pp_quad_strip")
+        torch.cuda.synchronize()
+        assert int(torch.count_nonzero(counts)) == 0
+        check([w[:, ::2] for w in wide], ref, f"call {rep}")
+        assert all(bool((w[:, 1::2] == 7.0).all()) for w in wide)
+    rc = L.pp_quad_strip(dc.data_ptr(), N, da.data_ptr(), K, ptrs, dt, nat.float_array(scales),
+                         nat.ptr_array([w.data_ptr() for w in wide]), 2 * N, 2, M, N, K, ws.data_ptr(), n_ws - 4,
+                         counts.data_ptr(), n_counts, torch.cuda.current_stream(DEV).cuda_stream)
+    assert rc == nat.PP_EINVAL
+
+
+def test_replayed_graph():
+    """A captured call replayed beside eager calls gives the eager outputs each time."""
+    K, N = 4096, 512
+    codes = u32(random_codes((K, N), 1)).to(DEV)
+    luts, scales = fp16_luts(1)
+    luts = [t.to(DEV) for t in luts]
+    for M in (1, 16):
+        a = torch.randn(M, K, device=DEV).half()
+        want = qk.quad_bitpacked(a, codes, luts, scales)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            got = qk.quad_bitpacked(a, codes, luts, scales)
+        for rep in range(4):
+            for t in got:
+                t.fill_(float("nan"))
+            g.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(x, y) for x, y in zip(got, want)), (M, rep)
+            again = qk.quad_bitpacked(a, codes, luts, scales)
+            assert all(torch.equal(x, y) for x, y in zip(again, want))
