@@ -389,6 +389,23 @@ int pp_quad_strip(const uint32_t* codes, int64_t ldk, const void* a, int64_t a_s
                   void* stream);
 
 /*
+ * Fused matrix-core decode of int16 (K,N) codes (stored = code ^ 0x8000, row stride ldk) for 1 to 32
+ * tokens, no plug table (polar_kernels.py:14-115); group of element (k, n): (k*N + n) / group_size:
+ *   pp_dual_strip_ok              1 if it reads these operands: K % 32 == 0, group_size a power of
+ *                                 two >= 4 that divides N, codes 8-byte aligned with ldk % 4 == 0,
+ *                                 activations 16-byte aligned with a_sm % 8 == 0, K * ldk < 2^29
+ *   pp_dual_strip_workspace_size  bytes of workspace (the K slices' float32 sums; any contents)
+ * Outputs (M,N) with row stride o_sm.
+ */
+int pp_dual_strip_ok(const void* codes, int64_t ldk, const void* a, int64_t a_sm, int64_t group_size, int64_t M,
+                     int64_t N, int64_t K);
+int64_t pp_dual_strip_workspace_size(int64_t M, int64_t N, int64_t K);
+int pp_dual_strip(const void* codes, int64_t ldk, const void* a, int64_t a_sm, const void* scales, int64_t group_size,
+                  const void* amp_lut, int64_t amp_n, const void* cos_lut, const void* sin_lut, int64_t phase_n,
+                  int lut_dtype, void* out1, void* out2, int64_t o_sm, int64_t M, int64_t N, int64_t K, void* workspace,
+                  int64_t workspace_bytes, void* stream);
+
+/*
  * The quad layer packer (pack_quad_layer, quad_kernels.py:16-50) over n tuples of four
  * equally laid out weight arrays w[m] (PP_F16 or PP_F32, aligned to 4 elements), on one stream:
  *   pp_quad_pack_squares  for each model, sq[i] = w[i]^2 in float32 (sq 16-byte aligned, its

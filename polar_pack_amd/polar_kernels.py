@@ -243,12 +243,22 @@ def dual_call_route(packed, M, *, layout="i16", group_size=32, chunk_size=0, ele
 
 def _dual_mfma(a, packed, bmax, amp_lut, cos_lut, sin_lut, num_phases, group_size, lut_dt, keep, pn, elem_base,
                out1, out2, L, dev):
-    """More than 8 tokens on the int16 (K,N) layout: the matrix-core decode (pp_dual_mfma).
+    """The matrix-core decodes of the int16 (K,N) layout: to 32 tokens without plug entries, with
+    groups that do not straddle rows, by strips of columns (pp_dual_strip), else pp_dual_mfma.
     Plug positions (k*ldk + n of the storage, relative to elem_base) move to the kernel's
     (N,K) frame n*K + k and are located per (column, K slice) (pp_plug_search)."""
     M, K = a.shape
     N = packed.shape[1]
     ldk = packed.stride(0)
+    if not pn and L.pp_dual_strip_ok(packed.data_ptr(), ldk, a.data_ptr(), a.stride(0), group_size, M, N, K):
+        ws_bytes = L.pp_dual_strip_workspace_size(M, N, K)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+        nat.check(L.pp_dual_strip(packed.data_ptr(), ldk, a.data_ptr(), a.stride(0), bmax.data_ptr(), group_size,
+                                  amp_lut.data_ptr(), amp_lut.numel(), cos_lut.data_ptr(), sin_lut.data_ptr(),
+                                  num_phases, lut_dt, out1.data_ptr(), out2.data_ptr(), out1.stride(0), M, N, K,
+                                  ws.data_ptr() if ws is not None else None, ws_bytes, nat.raw_stream(dev)),
+                  "pp_dual_strip")
+        return
     plan = (ctypes.c_int64 * 2)()
     nat.check(L.pp_dual_mfma_plan(M, N, K, ctypes.byref(plan, 0), ctypes.byref(plan, 8)), "pp_dual_mfma_plan")
     slices, cols = int(plan[0]), int(plan[1])
