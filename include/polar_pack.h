@@ -389,6 +389,21 @@ int pp_quad_strip(const uint32_t* codes, int64_t ldk, const void* a, int64_t a_s
                   void* stream);
 
 /*
+ * Fused matrix-core decode of (N,K) rows for 1 to 32 tokens (quad_kernels.py:103-159), the rows'
+ * plug entries found by the kernel (plug_idx ascending; positions as pp_quad_mfma's):
+ *   pp_quad_tile_ok              1 if it takes these sizes: K % 32 == 0, ldc >= K and % 4 == 0,
+ *                                a_sm % 8 == 0, at most 8 tiles of 16 rows a CU, plug_n < 2^28
+ *   pp_quad_tile_workspace_size  bytes of workspace (the K slices' float32 sums; any contents)
+ * codes and activations 16-byte aligned; outputs (M,N) with row stride o_sm.
+ */
+int pp_quad_tile_ok(int64_t ldc, int64_t a_sm, int64_t plug_n, int64_t M, int64_t N, int64_t K);
+int64_t pp_quad_tile_workspace_size(int64_t M, int64_t N, int64_t K);
+int pp_quad_tile(const uint32_t* codes, int64_t ldc, int64_t elem_base, const void* a, int64_t a_sm,
+                 const void* const* luts, int lut_dtype, const float* scales, const uint32_t* plug_idx,
+                 const void* plug_vals, int64_t plug_n, void* const* out, int64_t o_sm, int64_t M, int64_t N, int64_t K,
+                 void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * Fused matrix-core decode of int16 (K,N) codes (stored = code ^ 0x8000, row stride ldk) for 1 to 32
  * tokens, no plug table (polar_kernels.py:14-115); group of element (k, n): (k*N + n) / group_size:
  *   pp_dual_strip_ok              1 if it reads these operands: K % 32 == 0, group_size a power of

@@ -117,6 +117,9 @@ EXPORTS = {
     "pp_quad_strip_workspace_size": (i64, [i64, i64, i64]),
     "pp_quad_strip_counts": (i64, [i64, i64, i64]),
     "pp_quad_strip": (i32, [vp, i64, vp, i64, vp, i32, vp, vp, i64, i64, i64, i64, i64, vp, i64, vp, i64, vp]),
+    "pp_quad_tile_ok": (i32, [i64, i64, i64, i64, i64, i64]),
+    "pp_quad_tile_workspace_size": (i64, [i64, i64, i64]),
+    "pp_quad_tile": (i32, [vp, i64, i64, vp, i64, vp, i32, vp, vp, vp, i64, vp, i64, i64, i64, i64, vp, i64, vp]),
     "pp_dual_strip_ok": (i32, [vp, i64, vp, i64, i64, i64, i64, i64]),
     "pp_dual_strip_workspace_size": (i64, [i64, i64, i64]),
     "pp_dual_strip": (i32, [vp, i64, vp, i64, vp, i64, vp, i64, vp, vp, i64, i32, vp, vp, i64, i64, i64, i64, vp,

@@ -452,13 +452,24 @@ def _quad_prefill(a, codes, lut_ptrs, lut_dtype, sc, pi, pv, pn, elem_base, outs
 
 
 def _quad_mfma(a, codes, lut_ptrs, lut_dtype, sc, keep, pn, elem_base, outs, L, dev):
-    """5-64 tokens on (N,K) rows: the matrix-core batch decode (pp_quad_mfma), plug starts per
-    (row, K slice) found on the device (pp_plug_search; quaternion_packer.py:188-189)."""
+    """5-64 tokens on (N,K) rows: the matrix-core batch decode, to 32 tokens with rows dealt to
+    workgroups that find their plug entries themselves (pp_quad_tile), else (and past 8 tiles of
+    16 rows a CU) pp_quad_mfma with plug starts per (row, K slice) found on the device
+    (pp_plug_search; quaternion_packer.py:188-189)."""
     M, K = a.shape
     N = codes.shape[1]
     ldc = codes.stride(1)
     if a.stride(1) != 1 or a.data_ptr() % 16 or (M > 1 and a.stride(0) % 8):
         a = a.contiguous()
+    if L.pp_quad_tile_ok(ldc, a.stride(0), pn, M, N, K):
+        ws_bytes = L.pp_quad_tile_workspace_size(M, N, K)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+        nat.check(L.pp_quad_tile(codes.data_ptr(), ldc, elem_base, a.data_ptr(), a.stride(0), lut_ptrs, lut_dtype, sc,
+                                 keep[0].data_ptr() if pn else None, keep[1].data_ptr() if pn else None, pn,
+                                 nat.ptr_array([o.data_ptr() for o in outs]), outs[0].stride(0), M, N, K,
+                                 ws.data_ptr() if ws is not None else None, ws_bytes, nat.raw_stream(dev)),
+                  "pp_quad_tile")
+        return outs
     from .stream import mfma_slices
     slices, cols = mfma_slices(N, K, int(L.pp_quad_mfma_waves(M)))
     row_plug = None
