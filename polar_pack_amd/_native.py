@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import collections
 import ctypes as C
+import functools
 import os
 import threading
 
@@ -142,6 +143,8 @@ def lib_path() -> str:
 def lib() -> C.CDLL:
     """Load the HIP library once; raise if it is absent (no fallback path exists)."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is None:
             path = lib_path()
@@ -155,6 +158,13 @@ def lib() -> C.CDLL:
                 fn.argtypes = args
             _lib = h
     return _lib
+
+
+@functools.lru_cache(maxsize=4096)
+def sized(name: str, dev_index, *sizes: int) -> int:
+    """The library's size function ``name`` of these sizes on device ``dev_index`` (the answers
+    follow from the sizes and the device's CU count alone; ~1 us a call through ctypes)."""
+    return int(getattr(lib(), name)(*sizes))
 
 
 def check(rc: int, what: str) -> None:
@@ -248,7 +258,8 @@ def zero_workspace(dev, nbytes: int):
     import torch
     if nbytes <= 0:
         return None, None
-    dev = torch.device(dev)
+    if not isinstance(dev, torch.device):
+        dev = torch.device(dev)
     if torch.cuda.is_current_stream_capturing():
         return torch.zeros(nbytes, dtype=torch.uint8, device=dev), None
     key = (dev.index, raw_stream(dev))
@@ -257,10 +268,10 @@ def zero_workspace(dev, nbytes: int):
         if ws is None or ws.numel() < nbytes:
             ws = torch.zeros(max(nbytes, 1 << 16), dtype=torch.uint8, device=dev)
             _zero_ws[key] = ws
+            mine = [k for k in _zero_ws if k[0] == key[0] and k != key]
+            for k in mine[:max(0, len(mine) + 1 - ZERO_WS_STREAMS)]:
+                del _zero_ws[k]
         _zero_ws.move_to_end(key)
-        mine = [k for k in _zero_ws if k[0] == key[0]]
-        for k in mine[:max(0, len(mine) - ZERO_WS_STREAMS)]:
-            del _zero_ws[k]
     return ws, key
 
 

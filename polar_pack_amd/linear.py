@@ -46,8 +46,11 @@ class _PackedLinear(torch.nn.Module):
         lead = x.shape[:-1]
         if x.shape[-1] != self.in_features:
             raise ValueError(f"expected (..., {self.in_features}) input, got {tuple(x.shape)}")
-        outs = self._all(x.reshape(-1, self.in_features).to(torch.float16))
-        outs = [o.reshape(*lead, self.out_features) for o in outs]
+        if len(lead) == 1 and self.in_features and x.dtype == torch.float16:
+            outs = self._all(x)               # already (M, K) -> (M, N)
+        else:
+            outs = self._all(x.reshape(-1, self.in_features).to(torch.float16))
+            outs = [o.reshape(*lead, self.out_features) for o in outs]
         if self.bias is not None:
             outs = [o + self.bias for o in outs]
         return outs[self.model] if self.model is not None else tuple(outs)

@@ -236,9 +236,9 @@ def dual_call_route(packed, M, *, layout="i16", group_size=32, chunk_size=0, ele
     """The route (:data:`polar_pack_amd.routes.DUAL_ROUTES`) of a ``polar_dual_bitpacked`` call
     with these codes, M tokens and ``plug_n`` plug entries."""
     K, N = packed.shape
-    caps = routes.dual_storage(packed.stride(0), packed.stride(1), packed.data_ptr(), K, N, layout, group_size,
-                               chunk_size, int(elem_base), plug_n)
-    return routes.dual_route(M, K, N, caps, plug_n > 0, fused)
+    c_sk, c_sn = packed.stride()
+    return routes.dual_route_at(M, K, N, c_sk, c_sn, packed.data_ptr() % 16, layout, group_size, chunk_size,
+                                int(elem_base), plug_n, fused)
 
 
 def _dual_mfma(a, packed, bmax, amp_lut, cos_lut, sin_lut, num_phases, group_size, lut_dt, keep, pn, elem_base,
@@ -251,7 +251,7 @@ def _dual_mfma(a, packed, bmax, amp_lut, cos_lut, sin_lut, num_phases, group_siz
     N = packed.shape[1]
     ldk = packed.stride(0)
     if not pn and L.pp_dual_strip_ok(packed.data_ptr(), ldk, a.data_ptr(), a.stride(0), group_size, M, N, K):
-        ws_bytes = L.pp_dual_strip_workspace_size(M, N, K)
+        ws_bytes = nat.sized("pp_dual_strip_workspace_size", dev.index, M, N, K)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
         nat.check(L.pp_dual_strip(packed.data_ptr(), ldk, a.data_ptr(), a.stride(0), bmax.data_ptr(), group_size,
                                   amp_lut.data_ptr(), amp_lut.numel(), cos_lut.data_ptr(), sin_lut.data_ptr(),

@@ -229,8 +229,8 @@ def quad_call_route(codes, M, plug_n=0, fused=None):
     """The route (:data:`polar_pack_amd.routes.QUAD_ROUTES`) of a ``quad_bitpacked`` call with
     these codes, M tokens and ``plug_n`` plug entries."""
     K, N = codes.shape
-    caps = routes.quad_storage(codes.stride(0), codes.stride(1), codes.data_ptr(), K, N, plug_n)
-    return routes.quad_route(M, K, N, caps, plug_n > 0, fused)
+    c_sk, c_sn = codes.stride()
+    return routes.quad_route_at(M, K, N, c_sk, c_sn, codes.data_ptr() % 16, plug_n, fused)
 
 
 # Plans of the row kernel's one-Linear launches (pp_quad_rows): per plug table (the sorted
@@ -259,7 +259,7 @@ def _rows_plan(idx, pn, elem_base, ldc, M, N, K, L, dev):
         pos = idx.view(torch.int32).to(torch.int64) & 0xFFFFFFFF
         bounds = torch.tensor([elem_base, elem_base + (N - 1) * ldc + K], dtype=torch.int64, device=dev)
         lo, hi = (int(v) for v in torch.searchsorted(pos, bounds).tolist())
-    wave_plug = torch.empty(int(L.pp_quad_rows_plan_size(M)), dtype=torch.int64, device=dev)
+    wave_plug = torch.empty(nat.sized("pp_quad_rows_plan_size", dev.index, M), dtype=torch.int64, device=dev)
     if hi > lo:
         nat.check(L.pp_quad_rows_plan(idx.data_ptr() + 4 * lo, hi - lo, elem_base, ldc, M, N, K, wave_plug.data_ptr(),
                                       nat.raw_stream(dev)), "pp_quad_rows_plan")
@@ -285,7 +285,7 @@ def _quad_rows(a, codes, lut_ptrs, lut_dtype, sc, keep, pn, elem_base, outs, L, 
     wave_plug = None
     if pn:
         lo, hi, wave_plug = _rows_plan(keep[0], pn, elem_base, ldc, M, N, K, L, dev)
-    ws_bytes = L.pp_quad_rows_workspace_size(M, N, K)
+    ws_bytes = nat.sized("pp_quad_rows_workspace_size", dev.index, M, N, K)
     ws, wkey = nat.zero_workspace(dev, ws_bytes)
     n = hi - lo
     rc = L.pp_quad_rows(a.data_ptr(), a.stride(0), codes.data_ptr(), ldc, lut_ptrs, lut_dtype, sc,
@@ -328,9 +328,9 @@ def _quad_strip(a, codes, lut_ptrs, lut_dtype, sc, outs, L, dev):
     ldk, a_sm = codes.stride(0), a.stride(0)
     if not L.pp_quad_strip_ok(codes.data_ptr(), ldk, a.data_ptr(), a_sm, lut_dtype, M, N, K):
         return False
-    ws_bytes = L.pp_quad_strip_workspace_size(M, N, K)
+    ws_bytes = nat.sized("pp_quad_strip_workspace_size", dev.index, M, N, K)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    n_counts = L.pp_quad_strip_counts(M, N, K)
+    n_counts = nat.sized("pp_quad_strip_counts", dev.index, M, N, K)
     counts, wkey = nat.zero_workspace(dev, n_counts)
     rc = L.pp_quad_strip(codes.data_ptr(), ldk, a.data_ptr(), a_sm, lut_ptrs, lut_dtype, sc,
                          nat.ptr_array([o.data_ptr() for o in outs]), outs[0].stride(0), outs[0].stride(1), M, N, K,
@@ -461,8 +461,8 @@ def _quad_mfma(a, codes, lut_ptrs, lut_dtype, sc, keep, pn, elem_base, outs, L, 
     ldc = codes.stride(1)
     if a.stride(1) != 1 or a.data_ptr() % 16 or (M > 1 and a.stride(0) % 8):
         a = a.contiguous()
-    if L.pp_quad_tile_ok(ldc, a.stride(0), pn, M, N, K):
-        ws_bytes = L.pp_quad_tile_workspace_size(M, N, K)
+    if nat.sized("pp_quad_tile_ok", dev.index, ldc, a.stride(0), pn, M, N, K):
+        ws_bytes = nat.sized("pp_quad_tile_workspace_size", dev.index, M, N, K)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
         nat.check(L.pp_quad_tile(codes.data_ptr(), ldc, elem_base, a.data_ptr(), a.stride(0), lut_ptrs, lut_dtype, sc,
                                  keep[0].data_ptr() if pn else None, keep[1].data_ptr() if pn else None, pn,
