@@ -9,8 +9,11 @@
 // wavefront one tile x slice: 11008 x 2048 made 1,376 items for 2,048 wavefronts, 1.4 million
 // atomic adds and launches to find the rows' plug entries and to read the sums back.  Here a
 // wavefront finds its rows' entries itself while the LUTs travel, and one slice needs no second
-// launch.  What bounds it is the decode: ~17 vector instructions and 4 LDS reads (14 LDS clocks a
-// wavefront) a word, at two wavefronts a SIMD.
+// launch.  The decode takes ~19 vector instructions and 4 LDS reads (14 LDS clocks a wavefront) a
+// word; at two wavefronts a SIMD, all the tables leave room for, the vector units are busy 37 % and
+// LDS 21 % of the time (SQ counters), so what bounds it is the latency of a step's loads and lookups.
+// Per call in a graph (0.1 % plug), against quad_mfma_kernel: 11008 x 2048 at 5 / 16 tokens 46.3 / 49.4
+// -> 31.4 / 32.3 us; 4096 x 4096 38.1 / 38.7 -> 24.3 / 25.1; 2048 x 2048 28.5 / 24.7 -> 15.3 / 15.5.
 #include "quad_mfma.h"
 #include "slice_sums.h"
 
@@ -60,7 +63,9 @@ struct TileStage {
 };
 
 // The stage at column k of segment S.  Steps past the segment's end have resources of no bytes:
-// they read 0, cost no traffic and are not used.  Rows past N lie past the resource's end.
+// they read 0, cost no traffic and are not used.  Rows past N lie past the resource's end.  Two
+// loads share each 128-byte line, so the codes keep the caches' policy: with the streaming one
+// 11008 x 2048 at 16 tokens took 35.6 us for 32.3.
 template <int T>
 __device__ __forceinline__ void tile_issue(const QuadTileArgs& A, const TileSeg& S, int k, uint32_t voc,
                                            const uint32_t (&vox)[T], TileStage<T>& D) {
@@ -71,8 +76,8 @@ __device__ __forceinline__ void tile_issue(const QuadTileArgs& A, const TileSeg&
     const int kc = in ? k + 32 * u : 0;
     const rsrc_t rc = make_rsrc(A.codes + (int64_t)S.tile * 16 * A.ldc + kc,
                                 in ? 4u * (uint32_t)((int64_t)(nrows - 1) * A.ldc + (A.K - kc)) : 0u);
-    vload128(D.c[u][0], voc, rc);
-    vload128(D.c[u][1], voc + 16u, rc);
+    vload128c(D.c[u][0], voc, rc);
+    vload128c(D.c[u][1], voc + 16u, rc);
     const rsrc_t rx = make_rsrc(A.x + kc, in ? 2u * (uint32_t)((int64_t)(A.M - 1) * A.x_sm + (A.K - kc)) : 0u);
 #pragma unroll
     for (int t = 0; t < T; ++t) vload128c(D.xb[u][t], vox[t], rx);
