@@ -421,6 +421,23 @@ int pp_dual_strip(const void* codes, int64_t ldk, const void* a, int64_t a_sm, c
                   int64_t workspace_bytes, void* stream);
 
 /*
+ * Fused matrix-core decode of container (N,K) rows of pairs for 1 to 32 tokens, the rows' plug entries
+ * found by the kernel (plug_idx ascending stream positions):
+ *   pp_dual_tile_ok              1 if it takes these sizes: those of pp_dual_nk_mfma, and at most 8
+ *                                tiles of 16 rows a CU
+ *   pp_dual_tile_workspace_size  bytes of workspace (the K slices' float32 sums; any contents)
+ * codes and activations 16-byte aligned; outputs (M,N) with row stride o_sm.
+ */
+int pp_dual_tile_ok(int64_t ldc, int64_t elem_base, int64_t a_sm, int64_t group_size, int64_t chunk_size,
+                    int64_t plug_n, int64_t M, int64_t N, int64_t K);
+int64_t pp_dual_tile_workspace_size(int64_t M, int64_t N, int64_t K);
+int pp_dual_tile(const void* codes, int code_layout, int64_t ldc, int64_t elem_base, const void* a, int64_t a_sm,
+                 const void* scales, int64_t n_groups, int64_t group_size, int64_t chunk_size, const void* amp_lut,
+                 int64_t amp_n, const void* cos_lut, const void* sin_lut, int64_t phase_n, int lut_dtype,
+                 const uint32_t* plug_idx, const void* plug_amp, int64_t plug_n, void* out1, void* out2, int64_t o_sm,
+                 int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * The quad layer packer (pack_quad_layer, quad_kernels.py:16-50) over n tuples of four
  * equally laid out weight arrays w[m] (PP_F16 or PP_F32, aligned to 4 elements), on one stream:
  *   pp_quad_pack_squares  for each model, sq[i] = w[i]^2 in float32 (sq 16-byte aligned, its

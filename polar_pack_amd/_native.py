@@ -125,6 +125,10 @@ EXPORTS = {
     "pp_dual_strip_workspace_size": (i64, [i64, i64, i64]),
     "pp_dual_strip": (i32, [vp, i64, vp, i64, vp, i64, vp, i64, vp, vp, i64, i32, vp, vp, i64, i64, i64, i64, vp,
                             i64, vp]),
+    "pp_dual_tile_ok": (i32, [i64] * 9),
+    "pp_dual_tile_workspace_size": (i64, [i64, i64, i64]),
+    "pp_dual_tile": (i32, [vp, i32, i64, i64, vp, i64, vp, i64, i64, i64, vp, i64, vp, vp, i64, i32, vp, vp, i64, vp,
+                           vp, i64, i64, i64, i64, vp, i64, vp]),
     "pp_quad_pack_squares": (i32, [vp, i32, i64, vp, vp, vp]),
     "pp_quad_pack_norm": (i32, [vp, i32, i64, vp, vp, vp]),
     "pp_quad_pack_codes": (i32, [vp, i32, i64, f64, f64, vp, vp, vp]),

@@ -290,11 +290,24 @@ def _dual_mfma(a, packed, bmax, amp_lut, cos_lut, sin_lut, num_phases, group_siz
 
 def _dual_nk_mfma(a, packed, lay, scales, amp_lut, cos_lut, sin_lut, num_phases, group_size, chunk_size, lut_dt,
                   keep, pn, elem_base, out1, out2, L, dev):
-    """5-64 tokens on (N,K) container rows: the matrix-core decode (pp_dual_nk_mfma), plug
-    starts per (row, K slice) found on the device (pp_plug_search; polar_bitpack.py:240-243)."""
+    """(N,K) container rows on the matrix cores: to 32 tokens with rows dealt to workgroups that find
+    their plug entries themselves (pp_dual_tile), else (and past 8 tiles of 16 rows a CU)
+    pp_dual_nk_mfma, plug starts per (row, K slice) found on the device (pp_plug_search;
+    polar_bitpack.py:240-243)."""
     M, K = a.shape
     N = packed.shape[1]
     ldc = packed.stride(1)
+    if nat.sized("pp_dual_tile_ok", dev.index, ldc, elem_base, a.stride(0), group_size, chunk_size, pn, M, N, K):
+        ws_bytes = nat.sized("pp_dual_tile_workspace_size", dev.index, M, N, K)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+        nat.check(L.pp_dual_tile(packed.data_ptr(), lay, ldc, elem_base, a.data_ptr(), a.stride(0), scales.data_ptr(),
+                                 scales.numel(), group_size, chunk_size, amp_lut.data_ptr(), amp_lut.numel(),
+                                 cos_lut.data_ptr(), sin_lut.data_ptr(), num_phases, lut_dt,
+                                 keep[0].data_ptr() if pn else None, keep[1].data_ptr() if pn else None, pn,
+                                 out1.data_ptr(), out2.data_ptr(), out1.stride(0), M, N, K,
+                                 ws.data_ptr() if ws is not None else None, ws_bytes, nat.raw_stream(dev)),
+                  "pp_dual_tile")
+        return
     plan = (ctypes.c_int64 * 2)()
     nat.check(L.pp_dual_mfma_plan(M, N, K, ctypes.byref(plan, 0), ctypes.byref(plan, 8)), "pp_dual_mfma_plan")
     slices, cols = int(plan[0]), int(plan[1])
