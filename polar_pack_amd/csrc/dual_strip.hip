@@ -9,10 +9,9 @@
 // (plug tables, groups that straddle rows, more tokens) gives a wavefront 16 columns: it transposes
 // the weights through LDS and adds every slice's sums to memory by atomics.  What bounds both is
 // the decode, ~9 vector instructions and 2 LDS reads a code, and at these sizes the fixed cost of
-// a launch with its tables.  Per call in a graph, against dual_mfma_kernel: 4096 x 4096 at 2 / 8 /
-// 16 / 32 tokens 26.2 / 28.8 / 29.5 / 34.5 -> 18.3 / 17.4 / 18.3 / 20.8 us; K x N = 1536 x 11008 at
-// 8 / 32 tokens 33.4 / 42.5 -> 17.1 / 19.4; 11008 x 1536 30.5 / 36.5 -> 19.7 / 23.1; 512 x 512 at 8
-// tokens 13.9 -> 9.4.
+// a launch with its tables.  Per call in a graph, against dual_mfma_kernel: 4096 x 4096 at 8 / 32 tokens
+// 28.8 / 34.5 -> 15.4 / 19.2 us; K x N = 1536 x 11008 at 8 / 32 tokens 33.4 / 42.5 -> 15.6 / 18.2; 512 x
+// 512 at 8 tokens 13.9 -> 9.4.  Loads two, three or four steps ahead were slower (16.6 / 17.5 / 18.6 us).
 #include "dual_lds.h"
 #include "rows_common.h"
 #include "slice_sums.h"

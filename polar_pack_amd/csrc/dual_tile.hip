@@ -9,8 +9,8 @@
 // row (from the table itself where they do not fit): dual_nk_mfma_kernel reloads windows of 4 from
 // the table and waits for them nearly every step, and needs a launch before it to find the rows'
 // entries and one after it to read the atomics' sums.  Per call in a graph (1 % plug), against it:
-// 11008 x 2048 at 3 / 16 / 32 tokens 78.1 / 79.9 / 83.3 -> 34.6 / 36.0 / 37.1 us; 2048 x 11008 at 1 / 16
-// 58.0 / 59.3 -> 35.6 / 36.9; 4096 x 4096 at 16 46.5 -> 28.7; 1000 x 512 at 5 17.8 -> 12.1.
+// 11008 x 2048 at 3 / 16 / 32 tokens 78.1 / 79.9 / 83.3 -> 34.3 / 35.5 / 36.2 us; 2048 x 11008 at 1 / 16
+// 58.0 / 59.3 -> 34.5 / 36.2; 4096 x 4096 at 16 46.5 -> 28.4; 1000 x 512 at 5 17.8 -> 11.7.
 #include "dual_lds.h"
 #include "rows_common.h"
 #include "slice_sums.h"

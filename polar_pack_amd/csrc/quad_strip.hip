@@ -85,31 +85,33 @@ __device__ __forceinline__ HalfWord half_lookup(const char* lds, uint32_t cw, co
   return w;
 }
 
-// 16-byte units in address order: 16 per row; thread t writes unit t % 16 of rows t / 16 + 32 k.
+// Two threads an entry, 8 of the 16 units of 16 bytes of each of its rows a thread, neighbouring lanes
+// starting at different units (distinct banks).  7 loads a thread; with a unit's own values loaded by
+// the thread that writes it (32 loads) 4096 x 4096 took 19.5 us a call at 1 token (19.2 this way) and
+// the same at 32.
 struct HalfTables {
-  static constexpr int NT = QS_NT, KU = 4096 / NT;
-  uint32_t a[KU], b[KU];   // [norm | cos3, sin3] and [cos1, sin1 | cos2, sin2] rows
+  static_assert(QS_NT == 512, "two threads an entry");
+  uint32_t norm, t1, t2, t3;   // norm as float32, the (cos, sin) pairs
   __device__ __forceinline__ void load(const QuadLuts& L) {
-    const bool second = (threadIdx.x & 8) != 0;
-    const uint16_t* n = reinterpret_cast<const uint16_t*>(L.p[second ? 5 : 0]);
-    const uint16_t* s3 = reinterpret_cast<const uint16_t*>(L.p[second ? 6 : 0]);
-    const uint16_t* c = reinterpret_cast<const uint16_t*>(L.p[second ? 3 : 1]);
-    const uint16_t* s = reinterpret_cast<const uint16_t*>(L.p[second ? 4 : 2]);
+    const int e = threadIdx.x & 255;
+    uint32_t v[7];
 #pragma unroll
-    for (int k = 0; k < KU; ++k) {
-      const int e = (threadIdx.x >> 4) + NT / 16 * k;
-      a[k] = (uint32_t)n[e] | ((uint32_t)s3[e] << 16);
-      b[k] = (uint32_t)c[e] | ((uint32_t)s[e] << 16);
-    }
+    for (int i = 0; i < 7; ++i) v[i] = reinterpret_cast<const uint16_t*>(L.p[i])[e];
+    norm = v[0];
+    t1 = v[1] | (v[2] << 16);
+    t2 = v[3] | (v[4] << 16);
+    t3 = v[5] | (v[6] << 16);
   }
   __device__ __forceinline__ void store(char* lds) const {
-    const bool second = (threadIdx.x & 8) != 0;
+    const int e = threadIdx.x & 255;
+    const uint32_t n = __float_as_uint(h2f(norm));
 #pragma unroll
-    for (int k = 0; k < KU; ++k) {
-      const uint32_t va = second ? a[k] : __float_as_uint(h2f(a[k] & 0xFFFFu));
-      char* p = lds + 16 * (threadIdx.x + NT * k);
-      *reinterpret_cast<u32x4*>(p) = u32x4{va, va, va, va};
-      *reinterpret_cast<u32x4*>(p + 0x10000) = u32x4{b[k], b[k], b[k], b[k]};
+    for (int k = 0; k < 8; ++k) {
+      const int u = (k + 8 * (threadIdx.x >> 8) + e) & 15;
+      const uint32_t a = u < 8 ? n : t3, b = u < 8 ? t1 : t2;
+      char* p = lds + 256 * e + 16 * u;
+      *reinterpret_cast<u32x4*>(p) = u32x4{a, a, a, a};
+      *reinterpret_cast<u32x4*>(p + 0x10000) = u32x4{b, b, b, b};
     }
   }
 };

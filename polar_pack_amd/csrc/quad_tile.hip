@@ -13,7 +13,7 @@
 // word; at two wavefronts a SIMD, all the tables leave room for, the vector units are busy 37 % and
 // LDS 21 % of the time (SQ counters), so what bounds it is the latency of a step's loads and lookups.
 // Per call in a graph (0.1 % plug), against quad_mfma_kernel: 11008 x 2048 at 5 / 16 tokens 46.3 / 49.4
-// -> 31.4 / 32.3 us; 4096 x 4096 38.1 / 38.7 -> 24.3 / 25.1; 2048 x 2048 28.5 / 24.7 -> 15.3 / 15.5.
+// -> 30.8 / 31.9 us; 4096 x 4096 38.1 / 38.7 -> 24.1 / 24.6; 2048 x 2048 28.5 / 24.7 -> 14.6 / 15.4.
 #include "quad_mfma.h"
 #include "slice_sums.h"
 
