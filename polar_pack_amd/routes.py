@@ -19,7 +19,8 @@ Quad kernels (the reference's one fused kernel, quad_kernels.py:53-159, at every
                1-8 tokens (``pp_quad_gemm`` -> ``quad_rows_kernel``)
 * ``kn``       fused row decode of (K,N) codes with unit column stride (``pack_quad_layer``),
                8 tokens per pass (``pp_quad_gemm`` -> ``quad_kn_kernel``)
-* ``mfma``     matrix-core batch decode of (N,K) rows, 1-64 tokens per launch (``pp_quad_mfma``)
+* ``mfma``     matrix-core batch decode of (N,K) rows, 1-64 tokens per launch (``pp_quad_tile`` to
+               32 tokens, else ``pp_quad_mfma``)
 * ``big_nk``   fused matrix-core kernel on (N,K) rows, blocks of 16-256 tokens (``pp_quad_big``)
 * ``big_kn``   the same kernel on (K,N) codes as stored
 * ``kn_mfma``  (K,N) codes transposed into (N,K) rows, then ``mfma`` (``fused=False`` only)
@@ -28,10 +29,12 @@ Quad kernels (the reference's one fused kernel, quad_kernels.py:53-159, at every
 
 Dual kernels (polar_kernels.py:14-115):
 
-* ``dual_mfma``  matrix-core decode of the int16 (K,N) kernel layout (``pp_dual_mfma``)
+* ``dual_mfma``  matrix-core decode of the int16 (K,N) kernel layout (``pp_dual_strip`` to 32 tokens
+                 without plug entries, else ``pp_dual_mfma``)
 * ``dual_kn``    fused row decode of (K,N) codes, 8 tokens per pass (``pp_dual_gemm``)
 * ``dual_rows``  fused row decode of container (N,K) rows, 1-4 tokens (``pp_dual_gemm``)
-* ``dual_nk_mfma`` matrix-core decode of container (N,K) rows (``pp_dual_nk_mfma``)
+* ``dual_nk_mfma`` matrix-core decode of container (N,K) rows (``pp_dual_tile`` to 32 tokens, else
+                 ``pp_dual_nk_mfma``)
 * ``prefill`` / ``generic`` as for quad.
 
 The token boundaries are measured crossovers (graph-replayed GPU times on the reference's
@@ -83,7 +86,8 @@ def dual_mfma_min_m(K: int, N: int, has_plug: bool) -> int:
     row kernel, K x N = 11008x2048 30.2 / 31.5 / 32.1 against 33.8 / 37.9 / 40.6; at 1 token
     the row kernel wins, 21.8 against 25.2 us), else from 5 (2048x11008: 38.0 / 38.4 / 38.5
     against 29.6 / 34.6 / 38.1 us; with plug entries the matrix-core route moves them to its
-    frame on every call)."""
+    frame on every call).  Those are pp_dual_mfma's times; its strips take 18.3 us at 2 tokens and
+    4096x4096, and the calls below the bounds stay float32 so that they lose no precision."""
     return 2 if N <= K and not has_plug else 5
 
 
