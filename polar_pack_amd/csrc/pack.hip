@@ -88,12 +88,13 @@ __global__ __launch_bounds__(PK_NT) void quad_pack_norm_kernel(const Quad4 W, in
     float v[4][4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) load4<T>(W.w[m], i, n, v[m]);
-    // past n the weights read 0, which decides nothing unless a scale is 0: then every
-    // tuple's norm is NaN already
+    // only the tuples below n: the zeros past it would be 0 / 0 = NaN where a scale is 0, which
+    // weights whose squares underflow (a norm of w / 0 = infinity) must not become
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float x[4] = {v[0][e] / s[0], v[1][e] / s[1], v[2][e] / s[2], v[3][e] / s[3]};
-      top = max(top, __float_as_uint(quad_norm(x)) & 0x7FFFFFFFu);
+      const uint32_t norm = __float_as_uint(quad_norm(x)) & 0x7FFFFFFFu;
+      top = max(top, i + e < n ? norm : 0u);
     }
   }
   // one atomic a workgroup: one a wavefront (16,384 on one address) made this pass 200 us long

@@ -75,6 +75,17 @@ def test_quad_pack_is_the_tensor_expressions(monkeypatch, shape, kind, dtype):
     assert_same(got, want)
 
 
+@pytest.mark.parametrize("shape", [(1, 1), (3, 5), (2, 8), (1000, 777)])
+def test_quad_pack_of_weights_whose_squares_underflow(monkeypatch, shape):
+    """float32 weights of ~1e-25: a scale of 0, so norms of infinity, which the reads past an element
+    count that is no multiple of 4 must not turn into NaN."""
+    ws = [w * 1e-23 for w in weights(4, shape, torch.float32, "normal", 7)]
+    assert all(bool((w != 0).all()) and float((w.float() ** 2).mean()) == 0 for w in ws)
+    got, want = both(monkeypatch, qk.pack_quad_layer, *ws)
+    assert bool(want[1][0][1:].isinf().all())
+    assert_same(got, want)
+
+
 def test_quad_pack_keeps_a_transposed_layout(monkeypatch):
     ws = [w.t() for w in weights(4, (130, 64), torch.float16, "normal", 4)]
     got, want = both(monkeypatch, qk.pack_quad_layer, *ws)
