@@ -203,8 +203,8 @@ def raw_stream(dev) -> int:
 def packable(ws) -> bool:
     """Whether the packers' kernels may read these weights straight from memory: plain fp16 or
     float32 device tensors of one type, shape and stride order, dense and 16-byte aligned, with
-    no transform in force (tracing, vmap, forward-mode, autocast or a dispatch mode) that has to
-    see the tensor expressions themselves."""
+    no transform in force (tracing, vmap, forward-mode, autocast, a function or a dispatch mode) that
+    has to see the tensor expressions themselves."""
     import torch
     w0 = ws[0]
     if w0.device.type != "cuda" or w0.dtype not in (torch.float16, torch.float32) \
@@ -219,7 +219,8 @@ def packable(ws) -> bool:
                 or w.is_neg() or w.data_ptr() % 16:
             return False
     return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_autocast_enabled("cuda")
-                or torch._C._len_torch_dispatch_stack() or torch.autograd.forward_ad._current_level >= 0)
+                or torch._C._len_torch_function_stack() or torch._C._len_torch_dispatch_stack()
+                or torch.autograd.forward_ad._current_level >= 0)
 
 
 def upload(host, dev):

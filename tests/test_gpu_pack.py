@@ -122,3 +122,21 @@ def test_what_the_kernels_do_not_read_keeps_the_expressions(monkeypatch):
     many = torch.func.vmap(lambda x, y: pk.quantize_polar_bitpacked(x, y, group_size=32)[0])(
         torch.stack(w[:2]), torch.stack(w[2:]))
     assert many.shape == (2, *one[0].shape)
+
+
+def test_a_function_mode_sees_the_expressions():
+    class Seen(torch.overrides.TorchFunctionMode):
+        def __init__(self):
+            super().__init__()
+            self.names = set()
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.names.add(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    w = weights(4, (64, 96), torch.float32, "normal", 8)
+    for fn, ws in ((qk.pack_quad_layer, w), (pk.quantize_polar_bitpacked, w[:2])):
+        with Seen() as mode:
+            got = fn(*ws)
+        assert {"atan2", "log1p", "round"} <= mode.names, fn
+        assert_same(got, fn(*ws))
