@@ -454,11 +454,11 @@ int pp_quad_pack_codes(const void* const* w, int dtype, int64_t n, double mu, do
                        uint32_t* codes, void* stream);
 
 /*
- * bytes (a multiple of 4) of host memory to the device in the launch's own arguments: the
- * host memory is read before the call returns and nothing waits for earlier work.  For
- * tables of a few KB.  No counterpart in the reference.
+ * count tables, bytes[t] (a multiple of 4) of host memory at src[t] to device memory at dst[t], in the
+ * launches' own arguments (3,584 bytes a launch): the host memory is read before the call returns and
+ * nothing waits for earlier work.  For tables of a few KB.  No counterpart in the reference.
  */
-int pp_upload(void* dst, const void* src, int64_t bytes, void* stream);
+int pp_upload(void* const* dst, const void* const* src, const int64_t* bytes, int count, void* stream);
 
 /* ------------------------------------------------------------------------ */
 /* Dual pack: 16-bit [amp 6 | phase 10] -> 2 models.                          */

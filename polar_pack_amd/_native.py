@@ -133,7 +133,7 @@ EXPORTS = {
     "pp_quad_pack_norm": (i32, [vp, i32, i64, vp, vp, vp]),
     "pp_quad_pack_codes": (i32, [vp, i32, i64, f64, f64, vp, vp, vp]),
     "pp_dual_pack": (i32, [vp, vp, i32, i64, i64, i64, i32, f64, f64, vp, vp, vp]),
-    "pp_upload": (i32, [vp, vp, i64, vp]),
+    "pp_upload": (i32, [vp, vp, vp, i32, vp]),
 }
 
 _lock = threading.Lock()
@@ -223,14 +223,16 @@ def packable(ws) -> bool:
                 or torch.autograd.forward_ad._current_level >= 0)
 
 
-def upload(host, dev):
-    """A device copy of a small contiguous host tensor (a multiple of 4 bytes), carried in the
-    launches' arguments (pp_upload): unlike ``host.to(dev)`` it does not wait for queued work."""
+def upload(hosts, dev):
+    """Device copies of small contiguous host tensors (each a multiple of 4 bytes), every one with
+    storage of its own, carried in the launches' arguments (pp_upload): unlike ``host.to(dev)`` it
+    does not wait for queued work."""
     import torch
-    out = torch.empty(host.shape, dtype=host.dtype, device=dev)
-    check(lib().pp_upload(out.data_ptr(), host.data_ptr(), host.numel() * host.element_size(), raw_stream(dev)),
-          "pp_upload")
-    return out
+    outs = [torch.empty(h.shape, dtype=h.dtype, device=dev) for h in hosts]
+    sizes = (i64 * len(hosts))(*[h.numel() * h.element_size() for h in hosts])
+    check(lib().pp_upload(ptr_array([o.data_ptr() for o in outs]), ptr_array([h.data_ptr() for h in hosts]), sizes,
+                          len(hosts), raw_stream(dev)), "pp_upload")
+    return outs
 
 
 def plug_search(idx, n: int, pos0: int, pld: int, rows: int, slices: int, cols: int, dev):

@@ -230,12 +230,16 @@ __global__ __launch_bounds__(PK_NT) void dual_pack_kernel(const void* w1, const 
 // ------------------------------------------------------------------- host bytes to the device
 // A few KB of tables carried in the launch's own arguments: no staging buffer, and no wait
 // for the work queued before it, as a copy from pageable memory makes.
-constexpr int UP_WORDS = 896;
+constexpr int UP_WORDS = 896, UP_PARTS = 8;      // 3.7 KB of the 4 KB that a launch's arguments may take
 struct UpBlock {
   uint32_t v[UP_WORDS];
+  uint32_t* dst[UP_PARTS];
+  int first[UP_PARTS + 1];                       // part p: words first[p] .. first[p + 1] - 1
 };
-__global__ __launch_bounds__(PK_NT) void upload_kernel(const UpBlock B, uint32_t* dst, int n) {
-  for (int i = threadIdx.x; i < n; i += PK_NT) dst[i] = B.v[i];
+__global__ __launch_bounds__(PK_NT) void upload_kernel(const UpBlock B) {
+#pragma unroll
+  for (int p = 0; p < UP_PARTS; ++p)
+    for (int i = B.first[p] + threadIdx.x; i < B.first[p + 1]; i += PK_NT) B.dst[p][i - B.first[p]] = B.v[i];
 }
 
 static unsigned pack_grid(int64_t n, int per_thread, int per_cu = 16) {
@@ -328,17 +332,38 @@ extern "C" int pp_dual_pack(const void* w1, const void* w2, int dtype, int64_t n
   return PP_OK;
 }
 
-extern "C" int pp_upload(void* dst, const void* src, int64_t bytes, void* stream) {
-  PP_REQUIRE(bytes >= 0 && bytes % 4 == 0, "bytes must be a multiple of 4");
-  if (bytes == 0) return PP_OK;
-  PP_REQUIRE(dst != nullptr && src != nullptr && aligned(dst, 4), "null or misaligned pointer");
+extern "C" int pp_upload(void* const* dst, const void* const* src, const int64_t* bytes, int count, void* stream) {
+  PP_REQUIRE(count >= 0 && (count == 0 || (dst && src && bytes)), "null pointer argument");
+  for (int t = 0; t < count; ++t) {
+    PP_REQUIRE(bytes[t] >= 0 && bytes[t] % 4 == 0, "bytes must be a multiple of 4");
+    PP_REQUIRE(bytes[t] == 0 || (dst[t] != nullptr && src[t] != nullptr && aligned(dst[t], 4)),
+               "null or misaligned pointer");
+  }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const int64_t words = bytes / 4;
-  for (int64_t i = 0; i < words; i += UP_WORDS) {
-    const int n = (int)std::min<int64_t>(UP_WORDS, words - i);
+  int t = 0;
+  int64_t done = 0;                              // words of table t that earlier launches carry
+  while (t < count) {
     UpBlock B;
-    memcpy(B.v, reinterpret_cast<const char*>(src) + 4 * i, 4 * (size_t)n);
-    hipLaunchKernelGGL(upload_kernel, dim3(1), dim3(PK_NT), 0, st, B, reinterpret_cast<uint32_t*>(dst) + i, n);
+    int used = 0, parts = 0;
+    while (t < count && parts < UP_PARTS && used < UP_WORDS) {
+      const int64_t left = bytes[t] / 4 - done;
+      const int n = (int)std::min<int64_t>(UP_WORDS - used, left);
+      if (n > 0) {
+        memcpy(B.v + used, reinterpret_cast<const char*>(src[t]) + 4 * done, 4 * (size_t)n);
+        B.dst[parts] = reinterpret_cast<uint32_t*>(dst[t]) + done;
+        B.first[parts++] = used;
+        used += n;
+        done += n;
+      }
+      if (n == left) {
+        ++t;
+        done = 0;
+      }
+    }
+    if (used == 0) break;
+    for (int p = parts; p <= UP_PARTS; ++p) B.first[p] = used;
+    for (int p = parts; p < UP_PARTS; ++p) B.dst[p] = nullptr;
+    hipLaunchKernelGGL(upload_kernel, dim3(1), dim3(PK_NT), 0, st, B);
     PP_LAUNCH_CHECK();
   }
   return PP_OK;

@@ -84,10 +84,8 @@ def _layer_luts(levels, num_phases, mu, log_mu):
 
 @functools.lru_cache(maxsize=8)
 def _lut_block(levels, num_phases, mu, log_mu, default_dtype):
-    """[cos | sin | amp] of :func:`_layer_luts` as one host tensor (linspace follows torch's
-    default dtype, hence the key)."""
-    amp, cos, sin = _layer_luts(levels, num_phases, mu, log_mu)
-    return torch.cat([cos, sin, amp])
+    """:func:`_layer_luts` (linspace follows torch's default dtype, hence the key)."""
+    return _layer_luts(levels, num_phases, mu, log_mu)
 
 
 def _pack_on_device(w1, w2, amp_bits, num_phases, mu, group_size):
@@ -111,8 +109,8 @@ def _pack_dual_device(w1, w2, levels, num_phases, mu, log_mu, group_size):
                                          nat.PP_F16 if w1.dtype == torch.float16 else nat.PP_F32, n, group_size,
                                          num_phases, levels, mu, log_mu, packed.data_ptr(), bmax.data_ptr(),
                                          nat.raw_stream(dev)), "pp_dual_pack")
-        cos_lut, sin_lut, amp_lut = nat.upload(_lut_block(levels, num_phases, mu, log_mu, torch.get_default_dtype()),
-                                               dev).split([num_phases, num_phases, levels + 1])
+        amp_lut, cos_lut, sin_lut = nat.upload(_lut_block(levels, num_phases, mu, log_mu, torch.get_default_dtype()),
+                                               dev)
     return packed, bmax, amp_lut, cos_lut, sin_lut
 
 

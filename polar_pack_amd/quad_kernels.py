@@ -124,8 +124,8 @@ def _pack_quad_device(ws, mu):
         growth, rows = _lut_rows(mu)
         rows = rows.clone()
         rows[0] = growth * (top * 1.001) / mu
-        luts = nat.upload(rows, dev)
-    return codes.view(torch.uint32), list(luts.unbind(0)), scales
+        luts = nat.upload(list(rows.unbind(0)), dev)
+    return codes.view(torch.uint32), luts, scales
 
 
 def _lut_args(luts):

@@ -140,3 +140,24 @@ def test_a_function_mode_sees_the_expressions():
             got = fn(*ws)
         assert {"atan2", "log1p", "round"} <= mode.names, fn
         assert_same(got, fn(*ws))
+
+
+def test_luts_are_tensors_of_their_own():
+    """As the expressions' are: no two share storage or a version, so one can be changed in place,
+    saved or released by itself."""
+    w = weights(4, (64, 96), torch.float16, "normal", 9)
+    for luts in (qk.pack_quad_layer(*w)[1], pk.quantize_polar_bitpacked(*w[:2])[2:]):
+        assert len({t.untyped_storage().data_ptr() for t in luts}) == len(luts)
+        for t in luts:
+            assert not t._is_view() and t.untyped_storage().nbytes() == t.numel() * t.element_size()
+        luts[0].zero_()
+        assert [t._version for t in luts[1:]] == [luts[1]._version] * (len(luts) - 1) != [luts[0]._version]
+
+
+@pytest.mark.parametrize("sizes", [(1,), (896,), (897, 0, 5), (3, 2000, 1, 1), (1,) * 20, (0, 0)])
+def test_upload_of_several_tables(sizes):
+    """Tables that end inside, at and past a launch's 896 words, and more of them than its 8 parts."""
+    g = torch.Generator().manual_seed(sum(sizes))
+    hosts = [torch.randint(-2 ** 31, 2 ** 31 - 1, (n,), generator=g, dtype=torch.int32) for n in sizes]
+    for got, want in zip(nat.upload(hosts, DEV), hosts):
+        assert torch.equal(got.cpu(), want)
