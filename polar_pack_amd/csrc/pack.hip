@@ -10,8 +10,8 @@
 // instructions, so the code pass is bound by instruction issue (158 us for 4096 x 4096 tuples,
 // 129 us for 11008 x 2048 pairs).  One fused pass per dependence (squares -> norms -> codes)
 // replaces ~60 elementwise launches, each of them a pass over float32 or int64 intermediates:
-// a call takes 360 us for 4096 x 4096 tuples (2,311 us on the expressions) and 133 us for
-// 11008 x 2048 pairs (1,068 us).
+// a call, its LUTs built on the host under the passes, takes 364 us for 4096 x 4096 tuples (2,311 us
+// on the expressions) and 132 us for 11008 x 2048 pairs (1,068 us).
 #include "pp_common.h"
 
 #include <algorithm>
@@ -90,11 +90,12 @@ __global__ __launch_bounds__(PK_NT) void quad_pack_norm_kernel(const Quad4 W, in
     for (int m = 0; m < 4; ++m) load4<T>(W.w[m], i, n, v[m]);
     // only the tuples below n: the zeros past it would be 0 / 0 = NaN where a scale is 0, which
     // weights whose squares underflow (a norm of w / 0 = infinity) must not become
+    const int left = (int)min<int64_t>(n - i, 4);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float x[4] = {v[0][e] / s[0], v[1][e] / s[1], v[2][e] / s[2], v[3][e] / s[3]};
       const uint32_t norm = __float_as_uint(quad_norm(x)) & 0x7FFFFFFFu;
-      top = max(top, i + e < n ? norm : 0u);
+      top = max(top, e < left ? norm : 0u);
     }
   }
   // one atomic a workgroup: one a wavefront (16,384 on one address) made this pass 200 us long
@@ -236,10 +237,23 @@ struct UpBlock {
   uint32_t* dst[UP_PARTS];
   int first[UP_PARTS + 1];                       // part p: words first[p] .. first[p + 1] - 1
 };
+// One walk over the words of all parts, its loads side by side (a loop a part made the launch 5 us longer).
 __global__ __launch_bounds__(PK_NT) void upload_kernel(const UpBlock B) {
+  uint32_t v[(UP_WORDS + PK_NT - 1) / PK_NT];
 #pragma unroll
-  for (int p = 0; p < UP_PARTS; ++p)
-    for (int i = B.first[p] + threadIdx.x; i < B.first[p + 1]; i += PK_NT) B.dst[p][i - B.first[p]] = B.v[i];
+  for (int k = 0; k * PK_NT < UP_WORDS; ++k) v[k] = B.v[min((int)threadIdx.x + k * PK_NT, UP_WORDS - 1)];
+#pragma unroll
+  for (int k = 0; k * PK_NT < UP_WORDS; ++k) {
+    const int i = threadIdx.x + k * PK_NT;
+    uint32_t* dst = B.dst[0];
+    int at = i;
+#pragma unroll
+    for (int p = 1; p < UP_PARTS; ++p) {
+      dst = i >= B.first[p] ? B.dst[p] : dst;
+      at = i >= B.first[p] ? i - B.first[p] : at;
+    }
+    if (i < B.first[UP_PARTS]) dst[at] = v[k];
+  }
 }
 
 static unsigned pack_grid(int64_t n, int per_thread, int per_cu = 16) {

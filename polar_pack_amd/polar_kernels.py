@@ -24,7 +24,6 @@ torch.matmul).
 from __future__ import annotations
 
 import ctypes
-import functools
 import math
 
 import torch
@@ -82,12 +81,6 @@ def _layer_luts(levels, num_phases, mu, log_mu):
             torch.sin(phases).to(torch.float16))
 
 
-@functools.lru_cache(maxsize=8)
-def _lut_block(levels, num_phases, mu, log_mu, default_dtype):
-    """:func:`_layer_luts` (linspace follows torch's default dtype, hence the key)."""
-    return _layer_luts(levels, num_phases, mu, log_mu)
-
-
 def _pack_on_device(w1, w2, amp_bits, num_phases, mu, group_size):
     """Whether pack.hip's one-pass packer takes the call: weights it can read (row-major: groups
     run over the flattened layer), no gradient through the scales, codes that fit their fields and
@@ -109,8 +102,8 @@ def _pack_dual_device(w1, w2, levels, num_phases, mu, log_mu, group_size):
                                          nat.PP_F16 if w1.dtype == torch.float16 else nat.PP_F32, n, group_size,
                                          num_phases, levels, mu, log_mu, packed.data_ptr(), bmax.data_ptr(),
                                          nat.raw_stream(dev)), "pp_dual_pack")
-        amp_lut, cos_lut, sin_lut = nat.upload(_lut_block(levels, num_phases, mu, log_mu, torch.get_default_dtype()),
-                                               dev)
+        # the host's work while the pass runs
+        amp_lut, cos_lut, sin_lut = nat.upload(_layer_luts(levels, num_phases, mu, log_mu), dev)
     return packed, bmax, amp_lut, cos_lut, sin_lut
 
 

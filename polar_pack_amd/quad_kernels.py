@@ -26,7 +26,6 @@ from __future__ import annotations
 
 import collections
 import ctypes
-import functools
 import math
 import threading
 import weakref
@@ -70,26 +69,18 @@ def pack_quad_layer(w1, w2, w3, w4, mu=MU):
     q3 = torch.round(t3 / (2 * math.pi) * 255).clip(0, 255)
     codes = _u32_words(nq, q1, q2, q3)
     growth, angles = _lut_tables(mu)
-    luts = [t.to(w1.device) for t in ((growth * r_max / mu).to(torch.float16), *angles)]
+    luts = [t.to(torch.float16).to(w1.device) for t in (growth * r_max / mu, *angles)]
     return codes, luts, [float(sk) for sk in s]
 
 
 def _lut_tables(mu):
-    """What a layer's LUTs hold whatever its weights: exp(i/255 ln(1+mu)) - 1 in float32, which
-    r_max / mu scales to the norms, and the six fp16 angle tables (quad_kernels.py:39-49)."""
-    i = torch.arange(256, dtype=torch.float32)
-    half_turn = i / 255 * math.pi
-    full_turn = i / 255 * 2 * math.pi
-    angles = [torch.cos(half_turn), torch.sin(half_turn), torch.cos(half_turn), torch.sin(half_turn),
-              torch.cos(full_turn), torch.sin(full_turn)]
-    return torch.exp(i / 255 * math.log1p(mu)) - 1, [t.to(torch.float16) for t in angles]
-
-
-@functools.lru_cache(maxsize=8)
-def _lut_rows(mu):
-    """:func:`_lut_tables` as host tensors: the growth, and 7 fp16 rows whose first is the norms'."""
-    growth, angles = _lut_tables(mu)
-    return growth, torch.stack([torch.zeros_like(angles[0]), *angles])
+    """What a layer's LUTs hold whatever its weights, in float32: exp(i/255 ln(1+mu)) - 1, which
+    r_max / mu scales to the norms, and the six angle tables (quad_kernels.py:39-49)."""
+    u = torch.arange(256, dtype=torch.float32) / 255
+    half_turn = u * math.pi
+    full_turn = u * 2 * math.pi
+    cos, sin = torch.cos(half_turn), torch.sin(half_turn)
+    return torch.exp(u * math.log1p(mu)) - 1, (cos, sin, cos, sin, torch.cos(full_turn), torch.sin(full_turn))
 
 
 def _pack_quad_device(ws, mu):
@@ -119,12 +110,12 @@ def _pack_quad_device(ws, mu):
         known.record()
         nat.check(L.pp_quad_pack_codes(ptrs, dtype, n, mu, log_mu, meta.data_ptr(), codes.data_ptr(), stream),
                   "pp_quad_pack_codes")
+        # the host's work while the device's passes run (the two polar angles share their tables)
+        growth, (cos, sin, _, _, *turn) = _lut_tables(mu)
+        cos, sin, *turn = (t.to(torch.float16) for t in (cos, sin, *turn))
         known.synchronize()
         *scales, top = host.tolist()
-        growth, rows = _lut_rows(mu)
-        rows = rows.clone()
-        rows[0] = growth * (top * 1.001) / mu
-        luts = nat.upload(list(rows.unbind(0)), dev)
+        luts = nat.upload([(growth * (top * 1.001) / mu).to(torch.float16), cos, sin, cos, sin, *turn], dev)
     return codes.view(torch.uint32), luts, scales
 
 

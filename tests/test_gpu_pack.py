@@ -154,6 +154,18 @@ def test_luts_are_tensors_of_their_own():
         assert [t._version for t in luts[1:]] == [luts[1]._version] * (len(luts) - 1) != [luts[0]._version]
 
 
+def test_every_call_builds_its_own_tables(monkeypatch):
+    """Nothing of a packed layer is kept for the next call: the LUTs are computed in each."""
+    w = weights(4, (64, 96), torch.float16, "normal", 10)
+    for mod, name, fn, ws in ((qk, "_lut_tables", qk.pack_quad_layer, w),
+                              (pk, "_layer_luts", pk.quantize_polar_bitpacked, w[:2])):
+        calls = []
+        monkeypatch.setattr(mod, name, lambda *a, _f=getattr(mod, name): calls.append(1) or _f(*a))
+        for i in range(3):
+            fn(*ws)
+            assert len(calls) == i + 1, name
+
+
 @pytest.mark.parametrize("sizes", [(1,), (896,), (897, 0, 5), (3, 2000, 1, 1), (1,) * 20, (0, 0)])
 def test_upload_of_several_tables(sizes):
     """Tables that end inside, at and past a launch's 896 words, and more of them than its 8 parts."""
