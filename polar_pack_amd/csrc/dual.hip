@@ -60,6 +60,9 @@ struct DualGroup {
 constexpr int DR_NT = 512;       // threads per workgroup (one per CU: the tables take most of LDS)
 constexpr int DR_WAVES = DR_NT / 64;
 constexpr int DR_CHUNK = 512;    // pairs per wave, row and step: 8 per lane
+// Row strides from here on (a task's 8 rows then span 2^29 pairs, past which 32-bit byte offsets end)
+// take the form with a base a row.
+constexpr int64_t DR_WIDE = 1ll << 26;
 
 struct DualRowsArgs {
   const uint16_t* codes;   // code of (row 0, k 0)
@@ -79,46 +82,54 @@ struct DualRowsArgs {
   int64_t plug_n;
 };
 
-// A wave's task.  Its pairs are addressed by o = their offset from row0's first pair + low,
-// low being that pair's place in its group: pair o is in group o / gs of `scales` up to the
-// next chunk boundary, where the groups restart.
+// A wave's task.  Its pairs are addressed by o = their offset from a row's first pair + low, low
+// being that pair's place in its group: pair o is in group o / gs of `scales` up to the next chunk
+// boundary, where the groups restart.  The offsets are 32 bits: where a task's rows span more (WIDE)
+// each row has a base of its own, else row 0's serves them all (one division by the chunk size a task).
+template <int RG, bool WIDE>
 struct DrTask {
+  static constexpr int NB = WIDE ? RG : 1;
   int row0, nrows, k0, k1;
-  rsrc_t codes;            // the rows from k0 (past the last row's k1 it reads 0)
-  const f16* scales;       // the first pair's group scale
-  uint32_t low;
-  uint32_t edge;           // o of the next chunk boundary, 0xFFFFFFFF if past the task's rows
-  uint32_t edge_group;     // its group
+  rsrc_t codes[NB];        // the rows from k0 (past the last row's k1 it reads 0)
+  const f16* scales[NB];   // the first pair's group scale
+  uint32_t low[NB];
+  uint32_t edge[NB];       // o of the next chunk boundary, 0xFFFFFFFF if past the base's rows
+  uint32_t edge_group[NB]; // its group
 };
 
-template <int RG>
-__device__ __forceinline__ DrTask dr_task(const DualRowsArgs& A, int t, int part) {
-  DrTask T;
+template <int RG, bool WIDE>
+__device__ __forceinline__ DrTask<RG, WIDE> dr_task(const DualRowsArgs& A, int t, int part) {
+  DrTask<RG, WIDE> T;
   const int chunks = (A.K + DR_CHUNK - 1) / DR_CHUNK;
   T.row0 = min(t * RG, A.N);
   T.nrows = t < A.tasks ? min(RG, A.N - T.row0) : 0;
   T.k0 = (int)((int64_t)part * chunks / A.parts) * DR_CHUNK;
   T.k1 = min(A.K, (int)((int64_t)(part + 1) * chunks / A.parts) * DR_CHUNK);
   const bool any = T.nrows > 0 && T.k1 > T.k0;
-  T.codes = make_rsrc(A.codes + (int64_t)T.row0 * A.ldc + T.k0,
-                      any ? 2u * (uint32_t)((T.nrows - 1) * A.ldc + T.k1 - T.k0) : 0u);
-  const int64_t p = A.pos0 + (int64_t)T.row0 * A.ldc;
-  const int64_t c = p / A.grp.chunk, rem = p - c * A.grp.chunk, g = rem >> A.grp.log2gs;
-  T.scales = uniform_ptr(A.scales + c * A.grp.per_chunk + g);
-  T.low = (uint32_t)uniform((int)(rem & (A.grp.gs - 1)));
-  const int64_t edge = A.grp.chunk - (g << A.grp.log2gs);
-  const bool reaches = edge < (int64_t)T.low + RG * A.ldc;              // RG * ldc < 2^29
-  T.edge = (uint32_t)uniform(reaches ? (int)edge : -1);
-  T.edge_group = (uint32_t)uniform((int)(A.grp.per_chunk - g));
+#pragma unroll
+  for (int b = 0; b < DrTask<RG, WIDE>::NB; ++b) {
+    const int64_t at = (int64_t)(WIDE ? min(T.row0 + b, A.N - 1) : T.row0) * A.ldc;
+    const int64_t span = WIDE ? T.k1 - T.k0 : (T.nrows - 1) * A.ldc + T.k1 - T.k0;
+    T.codes[b] = make_rsrc(A.codes + at + T.k0, any && b < T.nrows ? 2u * (uint32_t)span : 0u);
+    const int64_t p = A.pos0 + at;
+    const int64_t c = p / A.grp.chunk, rem = p - c * A.grp.chunk, g = rem >> A.grp.log2gs;
+    T.scales[b] = uniform_ptr(A.scales + c * A.grp.per_chunk + g);
+    T.low[b] = (uint32_t)uniform((int)(rem & (A.grp.gs - 1)));
+    const int64_t edge = A.grp.chunk - (g << A.grp.log2gs);
+    const bool reaches = edge < (int64_t)T.low[b] + (WIDE ? A.K : RG * A.ldc);     // RG * ldc < 2^29, K < 2^30
+    T.edge[b] = (uint32_t)uniform(reaches ? (int)edge : -1);
+    T.edge_group[b] = (uint32_t)uniform((int)(A.grp.per_chunk - g));
+  }
   return T;
 }
 
-// Group of pair o.  Past the first boundary within the task a pair is d = o - edge pairs into
-// the following chunks; there are several only if a chunk is shorter than the task's rows.
-__device__ __forceinline__ uint32_t dr_group(const DualRowsArgs& A, const DrTask& T, uint32_t o) {
-  if (T.edge == 0xFFFFFFFFu) return o >> A.grp.log2gs;
-  if (o < T.edge) return o >> A.grp.log2gs;
-  uint32_t d = o - T.edge, g = T.edge_group;
+// Group of pair o of base b.  Past the first boundary within the task a pair is d = o - edge pairs into
+// the following chunks; there are several only if a chunk is shorter than the base's rows.
+template <int RG, bool WIDE>
+__device__ __forceinline__ uint32_t dr_group(const DualRowsArgs& A, const DrTask<RG, WIDE>& T, int b, uint32_t o) {
+  if (T.edge[b] == 0xFFFFFFFFu) return o >> A.grp.log2gs;
+  if (o < T.edge[b]) return o >> A.grp.log2gs;
+  uint32_t d = o - T.edge[b], g = T.edge_group[b];
   if (d >= A.grp.chunk) {
     const uint32_t q = d / (uint32_t)A.grp.chunk;
     d -= q * (uint32_t)A.grp.chunk;
@@ -141,19 +152,26 @@ struct DrStep {
 
 // A lane past the part's columns reads 0 for its pairs and activations, and the scale of the
 // part's last pairs (not used: dr_compute).
-template <int MT, int RG>
-__device__ __forceinline__ void dr_issue(const DualRowsArgs& A, const DrTask& T, const DrX<MT>& X, int k, int lane,
+template <int MT, int RG, bool WIDE>
+__device__ __forceinline__ void dr_issue(const DualRowsArgs& A, const DrTask<RG, WIDE>& T, const DrX<MT>& X, int k, int lane,
                                          DrStep<MT, RG>& S) {
   const int kk = k + 8 * lane, ld = (int)A.ldc;
   const bool in = kk < T.k1;
   const uint32_t voff = 2u * (uint32_t)(kk - T.k0);
 #pragma unroll
-  for (int r = 0; r < RG; ++r) vload128(S.q[r], in ? voff + 2u * (uint32_t)(r * ld) : OOB, T.codes);
-  const uint32_t o = T.low + (uint32_t)max(0, min(kk, T.k1 - 8));
+  for (int r = 0; r < RG; ++r) {
+    if constexpr (WIDE) vload128(S.q[r], in ? voff : OOB, T.codes[r]);
+    else vload128(S.q[r], in ? voff + 2u * (uint32_t)(r * ld) : OOB, T.codes[0]);
+  }
+  const uint32_t k8 = (uint32_t)max(0, min(kk, T.k1 - 8));
 #pragma unroll
   for (int r = 0; r < RG; ++r) {
-    const int row = max(0, min(r, T.nrows - 1));
-    S.sc[r] = T.scales[dr_group(A, T, o + (uint32_t)(row * ld))];
+    if constexpr (WIDE) {
+      S.sc[r] = T.scales[r][dr_group(A, T, r, T.low[r] + k8)];
+    } else {
+      const int row = max(0, min(r, T.nrows - 1));
+      S.sc[r] = T.scales[0][dr_group(A, T, 0, T.low[0] + k8 + (uint32_t)(row * ld))];
+    }
   }
 #pragma unroll
   for (int j = 0; j < MT; ++j) vload128c(S.x[j], in ? 2u * (uint32_t)kk : OOB, X.r[j]);
@@ -216,8 +234,8 @@ struct DrPlug {
   f16 x[MT];
 };
 
-template <int MT, int RG>
-__device__ __forceinline__ bool dr_plug_issue(const DualRowsArgs& A, const DrTask& T, int64_t e, uint32_t idx,
+template <int MT, int RG, bool WIDE>
+__device__ __forceinline__ bool dr_plug_issue(const DualRowsArgs& A, const DrTask<RG, WIDE>& T, int64_t e, uint32_t idx,
                                               DrPlug<MT>& P) {
   const int64_t pos = A.pos0 + (int64_t)T.row0 * A.ldc;
   const int64_t off = e < A.plug_n ? (int64_t)idx - pos : -1;
@@ -231,7 +249,13 @@ __device__ __forceinline__ bool dr_plug_issue(const DualRowsArgs& A, const DrTas
     if (k < A.K) {
       P.row = row;
       P.code = A.codes[(int64_t)(T.row0 + row) * A.ldc + k];
-      P.sc = T.scales[dr_group(A, T, T.low + (uint32_t)off)];
+      if constexpr (WIDE) {
+#pragma unroll
+        for (int r = 0; r < RG; ++r)
+          if (r == row) P.sc = T.scales[r][dr_group(A, T, r, T.low[r] + (uint32_t)k)];
+      } else {
+        P.sc = T.scales[0][dr_group(A, T, 0, T.low[0] + (uint32_t)off)];
+      }
       P.amp = A.plug_amp[e];
 #pragma unroll
       for (int j = 0; j < MT; ++j) P.x[j] = j < A.M ? A.x[(int64_t)j * A.x_sm + k] : (f16)0.f;
@@ -259,7 +283,7 @@ __device__ __forceinline__ void dr_plug_apply(const char* lds, const DualLane& d
   }
 }
 
-template <int MT, int RG, int LAYOUT>
+template <int MT, int RG, int LAYOUT, bool WIDE>
 __global__ __launch_bounds__(DR_NT) void dual_rows_kernel(const DualRowsArgs A) {
   constexpr int MP = MT == 3 ? 4 : MT;              // the reduction takes a power of two
   constexpr int NV = RG * 2 * MP, LNV = Log2<NV>::v;
@@ -272,13 +296,13 @@ __global__ __launch_bounds__(DR_NT) void dual_rows_kernel(const DualRowsArgs A) 
   DrX<MT> X;
 #pragma unroll
   for (int j = 0; j < MT; ++j) X.r[j] = make_rsrc(A.x + (int64_t)min(j, A.M - 1) * A.x_sm, j < A.M ? 2u * (uint32_t)A.K : 0u);
-  DrTask T;
+  DrTask<RG, WIDE> T;
   DrStep<MT, RG> s0, s1;
   int64_t e0 = 0;          // the lane's entry in the part's first window
   uint32_t idx0 = 0;
   auto task = [&](int round) {
-    T = dr_task<RG>(A, (int)blockIdx.x + (int)gridDim.x * (wave / parts + groups * round), part);
-    if (T.nrows > 0) dr_issue<MT, RG>(A, T, X, T.k0, lane, s0);
+    T = dr_task<RG, WIDE>(A, (int)blockIdx.x + (int)gridDim.x * (wave / parts + groups * round), part);
+    if (T.nrows > 0) dr_issue<MT, RG, WIDE>(A, T, X, T.k0, lane, s0);
   };
   auto window = [&]() {
     if (A.plug_n == 0 || T.nrows == 0) return;
@@ -311,18 +335,18 @@ __global__ __launch_bounds__(DR_NT) void dual_rows_kernel(const DualRowsArgs A) 
     if (T.nrows > 0) {
       // the task's entries, 64 a window, the windows dealt over its parts
       DrPlug<MT> P;
-      bool more = A.plug_n > 0 && dr_plug_issue<MT, RG>(A, T, e0, idx0, P);
+      bool more = A.plug_n > 0 && dr_plug_issue<MT, RG, WIDE>(A, T, e0, idx0, P);
       for (int k = T.k0; k < T.k1; k += 2 * DR_CHUNK) {
-        dr_issue<MT, RG>(A, T, X, k + DR_CHUNK, lane, s1);
+        dr_issue<MT, RG, WIDE>(A, T, X, k + DR_CHUNK, lane, s1);
         dr_compute<MT, RG, LAYOUT>(lds, dl, s0, k + 8 * lane < T.k1, acc);
         if (k + DR_CHUNK >= T.k1) break;
-        dr_issue<MT, RG>(A, T, X, k + 2 * DR_CHUNK, lane, s0);
+        dr_issue<MT, RG, WIDE>(A, T, X, k + 2 * DR_CHUNK, lane, s0);
         dr_compute<MT, RG, LAYOUT>(lds, dl, s1, k + DR_CHUNK + 8 * lane < T.k1, acc);
       }
       for (int64_t e = e0; more;) {
         dr_plug_apply<MT, RG, LAYOUT>(lds, dl, P, acc);
         e += 64 * parts;
-        more = dr_plug_issue<MT, RG>(A, T, e, A.plug_idx[min(e, A.plug_n - 1)], P);
+        more = dr_plug_issue<MT, RG, WIDE>(A, T, e, A.plug_idx[min(e, A.plug_n - 1)], P);
       }
     }
     float v[NV];
@@ -593,7 +617,7 @@ static bool dual_fast_ok(const void* a, int64_t a_sm, int64_t a_sk, const void* 
   return c_sk == 1 && c_sn % 8 == 0 && c_sn >= K && K % 8 == 0 && K > 0 && aligned(codes, 16) && M >= 1 &&
          M <= 4 && chunk > 0 && chunk % 8 == 0 && gs >= 8 && (gs & (gs - 1)) == 0 && elem_base % 8 == 0 &&
          (a_sk == 1 || K == 1) && (M == 1 || a_sm % 4 == 0) && aligned(a, 8) &&
-         c_sn < (1ll << 26);          // 32-bit offsets over a task's rows
+         K < (1ll << 30);             // 32-bit offsets in a row
 }
 
 struct DualRowsPlan {
@@ -603,12 +627,13 @@ struct DualRowsPlan {
 // Rows per task (8 or 4, from 3 tokens 4 or 2), parts of K per task (1, 2, 4 or 8 neighbouring
 // waves of a workgroup) and rounds of tasks.  Two costs decide, both in rows x chunks: what the
 // busiest workgroup decodes (its 8 waves share the CU's units) and what its slowest wave does
-// one after another, an item's reduction and stores counted as a chunk of 4 rows.
-static DualRowsPlan dual_rows_plan(int mt, int64_t N, int64_t K) {
+// one after another, an item's reduction and stores counted as a chunk of 4 rows.  Wide rows take the
+// smaller tasks, whose rows' bases stay in scalar registers.
+static DualRowsPlan dual_rows_plan(int mt, int64_t N, int64_t K, bool wide) {
   const int64_t chunks = (K + DR_CHUNK - 1) / DR_CHUNK, cus = device_cu_count();
   DualRowsPlan best = {};
   int64_t least = INT64_MAX;
-  for (int rg = mt <= 2 ? 8 : 4; rg >= (mt <= 2 ? 4 : 2); rg /= 2) {
+  for (int rg = (mt <= 2 ? 8 : 4) >> wide; rg >= (mt <= 2 ? 4 : 2); rg /= 2) {
     const int64_t tasks = (N + rg - 1) / rg;
     for (int parts = 1; parts <= DR_WAVES && parts <= chunks; parts *= 2) {
       const int64_t slots = cus * (DR_WAVES / parts), rounds = (tasks + slots - 1) / slots;
@@ -624,16 +649,24 @@ static DualRowsPlan dual_rows_plan(int mt, int64_t N, int64_t K) {
   return best;
 }
 
-template <int MT, int RG, int LAYOUT>
+template <int MT, int RG, int LAYOUT, bool WIDE = false>
 static int launch_dual_rows(const DualRowsArgs& A, hipStream_t st) {
-  hipLaunchKernelGGL((dual_rows_kernel<MT, RG, LAYOUT>), dim3((unsigned)std::min(device_cu_count(), A.tasks)),
+  hipLaunchKernelGGL((dual_rows_kernel<MT, RG, LAYOUT, WIDE>), dim3((unsigned)std::min(device_cu_count(), A.tasks)),
                      dim3(DR_NT), 0, st, A);
   PP_LAUNCH_CHECK();
   return PP_OK;
 }
 
 template <int LAYOUT>
-static int dispatch_dual_rows(const DualRowsArgs& A, int mt, int rg, hipStream_t st) {
+static int dispatch_dual_rows(const DualRowsArgs& A, int mt, int rg, bool wide, hipStream_t st) {
+  if (wide) {
+    switch (mt) {
+      case 1: return launch_dual_rows<1, 4, LAYOUT, true>(A, st);
+      case 2: return launch_dual_rows<2, 4, LAYOUT, true>(A, st);
+      case 3: return launch_dual_rows<3, 2, LAYOUT, true>(A, st);
+      default: return launch_dual_rows<4, 2, LAYOUT, true>(A, st);
+    }
+  }
   switch (mt) {
     case 1: return rg == 8 ? launch_dual_rows<1, 8, LAYOUT>(A, st) : launch_dual_rows<1, 4, LAYOUT>(A, st);
     case 2: return rg == 8 ? launch_dual_rows<2, 8, LAYOUT>(A, st) : launch_dual_rows<2, 4, LAYOUT>(A, st);
@@ -858,7 +891,8 @@ extern "C" int pp_dual_gemm(const void* a, int64_t a_sm, int64_t a_sk, const voi
   const DualLuts L = make_dual_luts(amp_lut, amp_lut_n, cos_lut, sin_lut, phase_n, lut_dtype);
   if (dual_fast_ok(a, a_sm, a_sk, codes, c_sk, c_sn, elem_base, chunk_size, group_size, M, K)) {
     const int mt = (int)M;
-    const DualRowsPlan p = dual_rows_plan(mt, N, K);
+    const bool wide = c_sn >= DR_WIDE;
+    const DualRowsPlan p = dual_rows_plan(mt, N, K, wide);
     DualRowsArgs A = {};
     A.codes = reinterpret_cast<const uint16_t*>(codes);
     A.ldc = c_sn;
@@ -885,8 +919,8 @@ extern "C" int pp_dual_gemm(const void* a, int64_t a_sm, int64_t a_sk, const voi
     A.plug_idx = plug_idx;
     A.plug_amp = reinterpret_cast<const f16*>(plug_amp);
     A.plug_n = plug_n;
-    return code_layout == PP_DUAL_U16_BE ? dispatch_dual_rows<PP_DUAL_U16_BE>(A, mt, p.rg, st)
-                                         : dispatch_dual_rows<PP_DUAL_I16_OFFSET>(A, mt, p.rg, st);
+    return code_layout == PP_DUAL_U16_BE ? dispatch_dual_rows<PP_DUAL_U16_BE>(A, mt, p.rg, wide, st)
+                                         : dispatch_dual_rows<PP_DUAL_I16_OFFSET>(A, mt, p.rg, wide, st);
   }
   if (dual_kn_ok(a, a_sm, a_sk, codes, c_sk, c_sn, group_size, chunk_size, std::min<int64_t>(M, 8), N, K)) {
     for (int64_t i0 = 0; i0 < M; i0 += 8) {

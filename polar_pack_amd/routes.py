@@ -219,7 +219,7 @@ def dual_storage(c_sk: int, c_sn: int, ptr: int, K: int, N: int, layout: str, gr
             caps.add("dual_pc")
     if c_sk == 1 and c_sn % 8 == 0 and c_sn >= K and K % 8 == 0 and K > 0 and a16 and chunk_size > 0 \
             and chunk_size % 8 == 0 and gs_ok and elem_base % 8 == 0:
-        if c_sn < 1 << 26:
+        if K < 1 << 30:
             caps.add("dual_rows")
         if K % 32 == 0 and 32 <= chunk_size < (1 << 30) and 32 * c_sn < (1 << 31) and N < (1 << 30) \
                 and plug_n < (1 << 29):

@@ -105,6 +105,9 @@ DUAL_TABLE = [
     (dict(dnk(2048, 512), chunk_size=24), (False, True), None, "dual_rows:1-4 prefill:5-"),   # chunks < 32 pairs
     (dnk(2056, 512), (False, True), None, "dual_rows:1-4 prefill:5-"),          # K % 32 != 0
     (dnk(2048, 512, elem_base=4), (False, True), None, "generic:1-4 prefill:5-"),
+    # rows 2^26 pairs and more apart: no 32-bit offset spans the matrix cores' 16 of them
+    (dict(dnk(2048, 512), c_sn=1 << 26), (False, True), None, "dual_rows:1-4 prefill:5-"),
+    (dict(dnk(2056, 512), c_sn=1 << 31), (False, True), None, "dual_rows:1-4 prefill:5-"),
     # K * ldk * 2 >= 2^31 bytes: neither the matrix cores nor the (K,N) kernel address it
     (dkn(16384, 65536), (False, True), None, "generic:1-4 prefill:5-"),
 ]
@@ -171,6 +174,17 @@ def test_dual_storage_matches_the_library():
                         assert DUAL_C[got] == r, (K, N, ptr, c_sk, c_sn, chunk, base, M, r, got)
                         n += 1
     assert n > 300
+
+
+def test_far_rows_match_the_library():
+    """Container rows of every stride are the row kernel's, in the route table and in the library."""
+    for ld in ((1 << 26) - 8, 1 << 26, (1 << 29) + 8, 1 << 31, 1 << 33):
+        for M in (1, 2, 3, 4):
+            for K in (8, 2056, (1 << 26) - 8):
+                caps = routes.dual_storage(1, ld, 256, K, 3, "u16be", 32, 50_000_000, 0)
+                assert routes.dual_route(M, K, 3, caps, False, fused=False) == "dual_rows", (ld, M, K)
+                got = nat.lib().pp_dual_gemm_kernel(4096, K, 1, 256, 1, ld, 32, 50_000_000, 0, M, 3, K)
+                assert got == nat.PP_GEMM_ROWS, (ld, M, K)
 
 
 def _u32(a):
