@@ -161,7 +161,11 @@ __device__ __forceinline__ void gemv_issue(const QuadStripArgs& A, int n0, int k
   for (int i = 0; i < 8; ++i) vload128(S.q[i], voff + 4u * (uint32_t)(i * A.ldk), rc);
 }
 
-__device__ __forceinline__ void gemv_compute(const char* lds, const HalfLane& hl, const GemvChunk& S, float (&acc)[16]) {
+// `in`: the lane's 8 rows lie in the wave's (its rows come in eights).  Rows past them are left out, not
+// multiplied as zeros: the tables' first entries need not be finite.
+__device__ __forceinline__ void gemv_compute(const char* lds, const HalfLane& hl, const GemvChunk& S, bool in,
+                                             float (&acc)[16]) {
+  if (!in) return;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const uint32_t xw = i < 2 ? S.x.x : i < 4 ? S.x.y : i < 6 ? S.x.z : S.x.w;
@@ -214,12 +218,12 @@ __global__ __launch_bounds__(QS_NT) void quad_strip_gemv_kernel(const QuadStripA
       for (int k = kb; k < ke; k += 2 * QG_ROWS) {
         gemv_issue(A, n0, k + QG_ROWS, ke, vo, lane, s1);
         __builtin_amdgcn_sched_barrier(0);
-        gemv_compute(lds, hl, s0, acc);
+        gemv_compute(lds, hl, s0, k + 8 * (lane >> 4) < ke, acc);
         __builtin_amdgcn_sched_barrier(0);
         if (k + QG_ROWS >= ke) break;
         gemv_issue(A, n0, k + 2 * QG_ROWS, ke, vo, lane, s0);
         __builtin_amdgcn_sched_barrier(0);
-        gemv_compute(lds, hl, s1, acc);
+        gemv_compute(lds, hl, s1, k + QG_ROWS + 8 * (lane >> 4) < ke, acc);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -326,6 +330,7 @@ struct StripWalk {
     xs(k + 32, xn);
     codes(k + 32, nxt);
     __builtin_amdgcn_sched_barrier(0);
+    if (k >= ke) return;               // no step of zeros: the tables' first entries need not be finite
     HalfWord w[2][8];
     look(cur, 0, w[0]);
 #pragma unroll
@@ -435,7 +440,7 @@ __global__ __launch_bounds__(QS_NT) void quad_strip_kernel(const QuadStripArgs A
 #pragma unroll
         for (int t = 0; t < TT; ++t) acc[c][m][t] = f4{0.f, 0.f, 0.f, 0.f};
     if (it < items) {
-      // two steps with no exit between them, so that each load stays in its step
+      // the loads of both steps with no exit between them, so that each load stays in its step
       for (int k = W.kb; k < W.ke; k += 64) {
         W.step(k, C0, C1, X0, X1, acc);
         W.step(k + 32, C1, C0, X1, X0, acc);

@@ -59,6 +59,24 @@ def test_matrix_core_tokens(K, N, ldk, M):
     check(got, kn_mfma_reference(a, wide[:, :N], luts, scales)[0], f"M={M}")
 
 
+@pytest.mark.parametrize("M", [1, 2, 16, 17, 32])
+@pytest.mark.parametrize("K,N", [(32, 8), (96, 300), (2080, 1000), (4128, 132), (64, 20_000)])
+def test_entries_no_code_names_do_not_matter(K, N, M):
+    """First table entries that are infinite or NaN, with no code 0 among the words: rows that a wave's
+    walk has no more of are left out, never decoded as zeros."""
+    words = random_codes((K, N), K + N + M) | np.uint32(0x01010101)
+    luts, scales = fp16_luts(K + M, split=M % 2 == 0)
+    a = torch.randn(M, K, device=DEV).half()
+    codes, dl = u32(words).to(DEV), [t.to(DEV) for t in luts]
+    want = qk.quad_bitpacked(a, codes, dl, scales, fused=True if M > 1 else None)
+    for bad in (float("inf"), float("nan")):
+        for t in dl:
+            t[0] = bad
+        got = qk.quad_bitpacked(a, codes, dl, scales, fused=True if M > 1 else None)
+        for m in range(4):
+            assert bool(want[m].isfinite().all()) and torch.equal(got[m], want[m]), (bad, m)
+
+
 @pytest.mark.parametrize("M", [1, 5, 20])
 def test_c_abi_workspace_and_strided_outputs(M):
     """Any workspace contents, counts zero before and after, outputs with a column stride, and the
