@@ -166,9 +166,9 @@ __global__ __launch_bounds__(DS_NT) void dual_strip_kernel(const DualStripArgs A
     for (int m = 0; m < 2; ++m)
 #pragma unroll
       for (int t = 0; t < TT; ++t) C[j][m][t] = f4{0.f, 0.f, 0.f, 0.f};
-  // two steps with no exit between them, so that each load stays in its step
   for (int k = kb; k < ke; k += 64) {
     W.step(k, S0, S1, C);
+    if (k + 32 >= ke) break;     // no step of zeros: the entries that a stored 0 names need not be finite
     W.step(k + 32, S1, S0, C);
   }
   __syncthreads();         // every wave is done with the tables

@@ -26,6 +26,25 @@ def test_matches_oracle(K, N, gs, M):
     check(outs, a, *arrs, gs, what=f"K={K} N={N} M={M}")
 
 
+@pytest.mark.parametrize("M", [1, 2, 16, 17, 32])
+@pytest.mark.parametrize("K,N,gs", [(32, 8, 8), (96, 72, 8), (2080, 192, 64), (64, 16_448, 32), (4128, 256, 256)])
+def test_entries_no_code_names_do_not_matter(K, N, gs, M):
+    """The entries that a stored 0 names infinite or NaN (amplitude 32, phase 0), no code naming them:
+    rows that a wave's walk has no more of are left out, never decoded as zeros."""
+    packed, bmax, *luts = layer(K, N, K + N + M, gs)
+    code = packed.view(np.uint16) ^ np.uint16(0x8000)
+    code = np.where(code >> 10 == 32, code ^ np.uint16(1 << 10), code) | np.uint16(1)
+    packed = (code ^ np.uint16(0x8000)).astype(np.uint16).view(np.int16)
+    a = np.random.default_rng(N + M).standard_normal((M, K)).astype(np.float16)
+    da, dp, db, amp, cos, sin = to_dev(a, packed, bmax, *luts)
+    want = pk.polar_dual_bitpacked(da, dp, db, amp, cos, sin, group_size=gs, fused=True)
+    for bad in (float("inf"), float("nan")):
+        amp[32] = cos[0] = sin[0] = bad
+        got = pk.polar_dual_bitpacked(da, dp, db, amp, cos, sin, group_size=gs, fused=True)
+        for o, w in zip(got, want):
+            assert bool(w.isfinite().all()) and torch.equal(o, w), bad
+
+
 @pytest.mark.parametrize("M", [1, 7, 20])
 def test_c_abi_strided_rows_and_workspace(M):
     """4-pair groups, float32 tables, rows of codes and outputs wider than N, any workspace."""
