@@ -1,5 +1,6 @@
 """GPU parity of the fused quad decode on the matrix cores (pp_quad_big: more than 64
-tokens, and 9-64 tokens on (K,N) storage, in blocks of 1, 2, 4 or 8 token tiles of 16;
+tokens, and 9-64 tokens on (K,N) storage, to 32 with a plug table or float32 tables
+(pp_quad_strip otherwise), in blocks of 1, 2, 4 or 8 token tiles of 16;
 forced with ``fused=True`` above the size where the drop-in operator switches to the fp16
 decode + library GEMM) against the float64 oracle: the fp16 operands the matrix cores
 multiply (the float32 decode rounded once, plug tuples substituted, as the reference's

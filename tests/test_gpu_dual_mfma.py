@@ -1,5 +1,6 @@
-"""GPU parity of the dual matrix-core decode (pp_dual_mfma, 2-64 tokens by default on the
-int16 (K,N) layout quantize_polar_bitpacked returns, from 5 when N > K or with plug entries) against the float64 oracle: the fp16
+"""GPU parity of the dual matrix-core decodes of the int16 (K,N) layout quantize_polar_bitpacked returns
+(2-64 tokens by default, from 5 when N > K or with plug entries; to 32 without plug entries and with
+groups that divide N the operator takes pp_dual_strip, else pp_dual_mfma) against the float64 oracle: the fp16
 operands the reference's tl.dot takes (the float32 decode (amp_lut * bmax) * cos/sin
 rounded once, plug amplitudes substituted, polar_kernels.py:60-82) within rel 1e-3 plus the
 float32 dot-product bound 2^-18 * sum |w x|, and normwise within 1e-3 of the exact decode."""
@@ -51,10 +52,10 @@ def test_kernel_layout_matches_oracle(K, N, plug, gs, M):
     """Several shapes (N not a multiple of 16, K = 96: one padded step), group sizes 8-64,
     plug amplitudes at random positions, 9-300 tokens (16-token tiles of 2, 4 or 8; one to
     two token blocks; K slices for the small batches), forced with fused=True above the
-    operator's default range.  Without plug entries and with N a multiple of 16 and of the
-    group size the kernel loads rows of 8 codes and transposes them through LDS (N = 400
-    with 32-pair groups takes the column loads); from 65 tokens those rows go to the
-    producer/consumer workgroups (64-column blocks: N = 208 ends in a partial block, K = 320
+    operator's default range.  Without plug entries and with N a multiple of the group size the
+    strips take them to 32 tokens (the one-wave form's row loads, which they stand for there:
+    test_row_loads_to_32_tokens); N = 400 with 32-pair groups, and 33-64 tokens, take the column
+    loads; from 65 tokens rows with N a multiple of 16 too go to the producer/consumer workgroups (64-column blocks: N = 208 ends in a partial block, K = 320
     in K slices of whole and partial super-steps; 128- and 256-token blocks)."""
     seed = K * 3 + N + plug + M + gs
     packed, bmax, amp_lut, cos_lut, sin_lut = layer(K, N, seed, gs)
@@ -132,6 +133,34 @@ def test_producer_consumer_float32_luts_odd_output_stride(M):
             assert bool(torch.isnan(w[:, N:]).all()), "a column past N was written"
     if ws_bytes:
         assert int(torch.count_nonzero(ws)) == 0, "the workspace is not left zero"
+
+
+@pytest.mark.parametrize("M", [2, 9, 16, 17, 32])
+@pytest.mark.parametrize("K,N,gs,ldk", [(1024, 384, 32, 384), (256, 512, 64, 512), (128, 64, 8, 64), (320, 208, 16, 208),
+                                        (256, 320, 32, 536), (4096, 96, 32, 96)])
+def test_row_loads_to_32_tokens(K, N, gs, ldk, M):
+    """pp_dual_mfma itself at the token counts where the operator takes pp_dual_strip (codes below 1 GiB):
+    rows of 8 codes transposed through LDS, rows wider than N, one and several K slices, an odd count
+    of steps a slice."""
+    packed_w, _, *luts = layer(K, ldk, K + N + M, gs if ldk == N else 8)
+    bmax = (np.random.default_rng(M).random(K * N // gs) * 0.5 + 0.05).astype(np.float16)
+    a = np.random.default_rng(K + M).standard_normal((M, K)).astype(np.float16)
+    L = nat.lib()
+    slices, cols = (ctypes.c_int64 * 1)(), (ctypes.c_int64 * 1)()
+    nat.check(L.pp_dual_mfma_plan(M, N, K, slices, cols), "pp_dual_mfma_plan")
+    s_, c_ = int(slices[0]), int(cols[0])
+    ws_bytes = L.pp_dual_mfma_workspace_size(M, N, s_)
+    ws = torch.zeros(max(ws_bytes, 16), dtype=torch.uint8, device=DEV)
+    da, dp, db, *dl = to_dev(a, packed_w, bmax, *luts)
+    outs = [torch.full((M, N), float("nan"), dtype=torch.float16, device=DEV) for _ in range(2)]
+    for rep in range(2):
+        nat.check(L.pp_dual_mfma(dp.data_ptr(), ldk, da.data_ptr(), K, db.data_ptr(), gs, dl[0].data_ptr(),
+                                 dl[0].numel(), dl[1].data_ptr(), dl[2].data_ptr(), dl[1].numel(), nat.PP_F16, None,
+                                 None, 0, None, 0, K, s_, c_, outs[0].data_ptr(), outs[1].data_ptr(), N, M, N, K,
+                                 ws.data_ptr(), ws_bytes, nat.raw_stream(DEV)), "pp_dual_mfma")
+        torch.cuda.synchronize()
+        check(outs, a, packed_w[:, :N], bmax, *luts, gs, None, f"K={K} N={N} M={M} rep={rep}")
+    assert ws_bytes == 0 or int(torch.count_nonzero(ws)) == 0
 
 
 @pytest.mark.parametrize("M", [20, 70])

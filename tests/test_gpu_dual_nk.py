@@ -1,9 +1,12 @@
-"""GPU parity of the matrix-core dual decode over .dualpack container rows (pp_dual_nk_mfma:
-5-64 tokens by default, any size with ``fused=True``) against the float64 oracle
+"""GPU parity of the matrix-core dual decodes over .dualpack container rows (the operator: pp_dual_tile
+to 32 tokens, pp_dual_nk_mfma above, any size with ``fused=True``; pp_dual_nk_mfma to 32 tokens through
+the C ABI) against the float64 oracle
 (oracle.dualpack.decode_pairs_f64, the restatement of unpack_dual_models,
 polar_bitpack.py:228-247): weights rounded to fp16 before the product, as the reference's
 kernel rounds them (polar_kernels.py:78-82), so the outputs are held to the fp16-weight
 bound and normwise 1e-3 of the exact products."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -122,6 +125,46 @@ def test_workspace_left_zero_and_repeatable():
     check(a.cpu().numpy(), [torch.from_numpy(r) for r in res[0]], (d1.reshape(N, K), d2.reshape(N, K)), "C-ABI")
     for m in range(2):
         np.testing.assert_allclose(res[1][m], res[0][m], rtol=2e-3, atol=2e-3)
+
+
+@pytest.mark.parametrize("layout", ["u16be", "i16"])
+@pytest.mark.parametrize("M", [1, 5, 16, 17, 32])
+@pytest.mark.parametrize("N,K,chunk,gs,cap,pos", [(96, 512, 4096, 32, 0.02, 0), (70, 1024, 1000, 64, 0.03, 0),
+                                                  (33, 256, 50_000_000, 32, 0.0, 0), (128, 2048, 2048, 8, 0.01, 0),
+                                                  (48, 800, 3000, 32, 0.03, 56_008)])
+def test_c_abi_to_32_tokens(N, K, chunk, gs, cap, pos, M, layout):
+    """pp_dual_nk_mfma itself at the token counts where the operator takes pp_dual_tile up to 8 tiles of
+    16 rows a CU: chunks that end inside rows, 8- to 64-pair groups, ragged N, a projection mid-stream,
+    no plug table, both code layouts, and the K slices of the plan."""
+    dp = pack(pos + N * K + 900, pos + N * K + 300, 300 + N + M, cap, chunk, gs)
+    amp, cs, sn = pk.header_luts(mu=dp.mu, device=DEV)
+    codes = be_codes_tensor(dp)
+    lay = nat.PP_DUAL_U16_BE
+    if layout == "i16":
+        v = codes.view(torch.int16).int() & 0xFFFF
+        codes, lay = ((((v & 0xFF) << 8) | (v >> 8)) - 32768).short(), nat.PP_DUAL_I16_OFFSET
+    codes = codes[pos:pos + N * K].clone()
+    scales = torch.from_numpy(dp.scales).to(DEV)
+    idx, val = u32(dp.plug_idx).to(DEV), torch.from_numpy(dp.plug_val).to(DEV)
+    pn, L = idx.numel(), nat.lib()
+    slices, cols = (ctypes.c_int64 * 1)(), (ctypes.c_int64 * 1)()
+    nat.check(L.pp_dual_mfma_plan(M, N, K, slices, cols), "pp_dual_mfma_plan")
+    s_, c_ = int(slices[0]), int(cols[0])
+    row_plug = nat.plug_search(idx, pn, pos, K, N, s_, c_, DEV) if pn else None
+    ws_bytes = L.pp_dual_mfma_workspace_size(M, N, s_)
+    ws = torch.zeros(max(ws_bytes, 16), dtype=torch.uint8, device=DEV)
+    a = np.random.default_rng(M).standard_normal((M, K)).astype(np.float16)
+    da = torch.from_numpy(a).to(DEV)
+    outs = [torch.full((M, N + 8), 7.0, dtype=torch.float16, device=DEV) for _ in range(2)]
+    nat.check(L.pp_dual_nk_mfma(codes.data_ptr(), lay, K, pos, da.data_ptr(), K, scales.data_ptr(), scales.numel(), gs,
+                                chunk, amp.data_ptr(), amp.numel(), cs.data_ptr(), sn.data_ptr(), cs.numel(),
+                                nat.PP_F32, idx.data_ptr() if pn else None, val.data_ptr() if pn else None, pn,
+                                row_plug.data_ptr() if pn else None, s_, c_, outs[0].data_ptr(), outs[1].data_ptr(),
+                                N + 8, M, N, K, ws.data_ptr(), ws_bytes, nat.raw_stream(DEV)), "pp_dual_nk_mfma")
+    torch.cuda.synchronize()
+    ref = [w.reshape(N, K) for w in odp.decode_pairs_f64(dp, pos, pos + N * K)]
+    check(a, [o[:, :N] for o in outs], ref, f"N={N} K={K} M={M} {layout}")
+    assert all(bool((o[:, N:] == 7.0).all()) for o in outs)
 
 
 def test_rejects_unaligned_rows():

@@ -27,6 +27,30 @@ def test_matches_oracle(N, K, chunk, cap, M):
     check(a, outs, ws, f"{N}x{K} M={M}")
 
 
+@pytest.mark.parametrize("M", [2, 16, 32])
+@pytest.mark.parametrize("N,K,chunk", [(680, 2816, 50_000_000), (1500, 4096, 9000)])
+def test_several_slices_of_several_tiles(N, K, chunk, M):
+    """Two and three tiles a workgroup, each in slices of K."""
+    pos, tiles = 56, -(-N // 16)
+    dp = pack(pos + N * K + 40, pos + N * K + 8, N, 0.01, chunk)
+    slices = nat.lib().pp_dual_tile_workspace_size(M, N, K) // (8 * M * 16 * tiles)
+    assert slices > 1 and tiles > torch.cuda.get_device_properties(DEV).multi_processor_count // slices
+    route, a, outs, ws = run(dp, pos, N, K, M, fused=True)
+    assert route == "dual_nk_mfma"
+    check(a, outs, ws, f"{N}x{K} M={M}")
+
+
+@pytest.mark.parametrize("M", [3, 17, 32])
+def test_rows_past_eight_tiles_a_cu(M):
+    """A head's row count stays on pp_dual_nk_mfma (search, atomics, finish)."""
+    N, K, pos, chunk = 16 * 8 * torch.cuda.get_device_properties(DEV).multi_processor_count + 21, 64, 56, 4104
+    dp = pack(pos + N * K + 40, pos + N * K + 8, N, 0.02, chunk)
+    assert not nat.lib().pp_dual_tile_ok(K, pos, K, 32, chunk, int(dp.plug_idx.size), M, N, K)
+    route, a, outs, ws = run(dp, pos, N, K, M, fused=True)
+    assert route == "dual_nk_mfma"
+    check(a, outs, ws, f"{N}x{K} M={M}")
+
+
 @pytest.mark.parametrize("M", [3, 20])
 def test_more_entries_than_lds_holds(M):
     N, K = 4100, 1024          # four steps of 16 x 32 pairs a wavefront, over half of them plugged

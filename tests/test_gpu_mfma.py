@@ -108,7 +108,7 @@ def test_dense_plug_rows_refill_the_window():
 
 @pytest.mark.parametrize("M", [12, 64, 100, 130, 300])
 def test_drop_in_operator_takes_the_matrix_cores_for_large_batches(M):
-    """9..64 tokens in one launch of the batch decode, 65..128 on the fused large-batch
+    """5..32 tokens on the tile kernel, 33..64 in one launch of the batch decode, 65..128 on the fused large-batch
     kernel (both multiply the fp16-rounded decode on the matrix cores); more (the
     reference's prefill sizes) as an fp16 decode of the (N,K) storage and a library GEMM."""
     qp, pack = packed(SHAPES, 35, threshold=0.015)

@@ -34,6 +34,37 @@ def test_matches_oracle(N, K, M):
     check(got, oracle(qp, pos, N, K, x), f"{N}x{K} M={M}")
 
 
+@pytest.mark.parametrize("M", [5, 16, 32])
+@pytest.mark.parametrize("N,K", [(680, 2816), (1500, 4096)])
+def test_several_slices_of_several_tiles(N, K, M):
+    """Two and three tiles a workgroup, each in slices of K."""
+    qp, pack = packed([(3, 40), (N, K), (2, 36)], 7, threshold=0.015)
+    pos, tiles = 120, -(-N // 16)
+    slices = nat.lib().pp_quad_tile_workspace_size(M, N, K) // (16 * M * 16 * tiles)
+    assert slices > 1 and tiles > torch.cuda.get_device_properties(DEV).multi_processor_count // slices
+    x = np.random.default_rng(N + M).standard_normal((M, K)).astype(np.float16)
+    codes = pack.codes[pos:pos + N * K].reshape(N, K).t()
+    luts = [t.to(DEV) for t in qk.header_luts(qp.r_max)]
+    got = qk.quad_bitpacked(torch.from_numpy(x).to(DEV), codes, luts, list(qp.s), plug=(pack.plug_idx, pack.plug_vals),
+                            elem_base=pos)
+    check(got, oracle(qp, pos, N, K, x), f"{N}x{K} M={M}")
+
+
+@pytest.mark.parametrize("M", [5, 17, 32])
+def test_rows_past_eight_tiles_a_cu(M):
+    """A head's row count stays on pp_quad_mfma (search, atomics, finish)."""
+    N, K = 16 * 8 * torch.cuda.get_device_properties(DEV).multi_processor_count + 21, 64
+    qp, pack = packed([(3, 40), (N, K), (2, 36)], 7, threshold=0.015)
+    pos = 120
+    assert not nat.lib().pp_quad_tile_ok(K, K, int(pack.plug_idx.numel()), M, N, K)
+    codes = pack.codes[pos:pos + N * K].reshape(N, K).t()
+    assert qk.quad_call_route(codes, M, 1) == "mfma"
+    x = np.random.default_rng(N + M).standard_normal((M, K)).astype(np.float16)
+    got = qk.quad_bitpacked(torch.from_numpy(x).to(DEV), codes, [t.to(DEV) for t in qk.header_luts(qp.r_max)],
+                            list(qp.s), plug=(pack.plug_idx, pack.plug_vals), elem_base=pos)
+    check(got, oracle(qp, pos, N, K, x), f"{N}x{K} M={M}")
+
+
 @pytest.mark.parametrize("M,share", [(8, 0.0), (16, 0.3), (32, 0.3)])
 @pytest.mark.parametrize("split", [False, True])
 def test_dense_plugs_strided_rows_and_workspace(M, share, split):

@@ -9,7 +9,7 @@ import torch
 from parity import assert_gemv_close, normwise
 from polar_pack_amd import _native as nat
 from polar_pack_amd import quad_kernels as qk
-from refs import kn_mfma_reference
+from refs import check_mfma, kn_mfma_reference
 from test_gpu_big import fp16_luts, random_codes, u32
 
 pytestmark = pytest.mark.gpu
@@ -75,6 +75,49 @@ def test_entries_no_code_names_do_not_matter(K, N, M):
         got = qk.quad_bitpacked(a, codes, dl, scales, fused=True if M > 1 else None)
         for m in range(4):
             assert bool(want[m].isfinite().all()) and torch.equal(got[m], want[m]), (bad, m)
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 2112, 8308), (16, 3648, 8308), (32, 5952, 4148)])
+def test_several_slices_and_rounds(M, K, N):
+    """More items of strips x slices than CUs: a workgroup's second item after a slice that was not its
+    strip's last, the buffers and the count's flag used again.  64 columns and the ragged last strip."""
+    cols = np.unique(np.concatenate([np.random.default_rng(M).choice(N, 48, replace=False), np.arange(N - 16, N)]))
+    words = random_codes((K, N), K + N + M)
+    luts, scales = fp16_luts(K + M)
+    a = np.random.default_rng(N + M).standard_normal((M, K)).astype(np.float16)
+    width, cus = 32 if M > 16 else 64, torch.cuda.get_device_properties(DEV).multi_processor_count
+    strips = -(-N // width)
+    slices, rest = divmod(nat.lib().pp_quad_strip_workspace_size(M, N, K), 16 * M * strips * width)
+    assert slices > 1 and rest == 0 and strips * slices > cus
+    da, dc, dl = torch.from_numpy(a).to(DEV), u32(words).to(DEV), [t.to(DEV) for t in luts]
+    exact = kn_mfma_reference(a, words, luts, scales, cols=cols)[0]
+    first = None
+    for rep in range(3):
+        got = qk.quad_bitpacked(da, dc, dl, scales, fused=True if M > 1 else None)
+        torch.cuda.synchronize()
+        first = first or got
+        assert all(torch.equal(g, f) for g, f in zip(got, first)), rep
+    check([g[:, torch.from_numpy(cols).to(DEV)] for g in first], exact, f"M={M}")
+
+
+@pytest.mark.parametrize("M", [1, 2, 16, 17, 32])
+@pytest.mark.parametrize("K,N", [(256, 72), (2080, 1000)])
+def test_float32_tables_keep_the_other_kernels(K, N, M):
+    """Tables that fp16 does not hold: quad_kn_kernel at one token, quad_big_kernel above."""
+    words = random_codes((K, N), K + N + M)
+    luts, scales = fp16_luts(K + M, split=M % 2 == 0)
+    luts = [t.float() * (1 + 2.0 ** -14) for t in luts]
+    a = np.random.default_rng(N + M).standard_normal((M, K)).astype(np.float16)
+    codes = u32(words).to(DEV)
+    assert not nat.lib().pp_quad_strip_ok(codes.data_ptr(), N, 0, K, nat.PP_F32, M, N, K)
+    got = qk.quad_bitpacked(torch.from_numpy(a).to(DEV), codes, [t.to(DEV) for t in luts], scales,
+                            fused=True if M > 1 else None)
+    ref = kn_mfma_reference(a, words, luts, scales)
+    if M > 1:
+        check_mfma(got, ref, f"M={M}")
+        return
+    for m in range(4):
+        assert_gemv_close(got[m].float().cpu().numpy(), ref[0][m], f"model {m}", rtol=5.1e-4)
 
 
 @pytest.mark.parametrize("M", [1, 5, 20])
