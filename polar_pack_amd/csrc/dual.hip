@@ -26,13 +26,6 @@
 
 namespace pp {
 
-// 16-bit word as stored -> code (amp << 10 | phase)
-template <int LAYOUT>
-__device__ __forceinline__ uint32_t dual_code(uint32_t half16) {
-  if constexpr (LAYOUT == PP_DUAL_U16_BE) return ((half16 & 0xFFu) << 8) | (half16 >> 8);
-  else return half16 ^ 0x8000u;
-}
-
 struct DualGroup {
   int64_t gs, chunk;  // chunk == 0: logical (k*N + n) // gs of a (K,N) matrix
   int64_t per_chunk;  // ceil(chunk / gs)

@@ -58,10 +58,6 @@ __device__ __forceinline__ float lut_at(const void* p, int dtype, int i) {
                          : reinterpret_cast<const float*>(p)[i];
 }
 
-__device__ __forceinline__ u32x4 load_nt(const uint32_t* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-}
-
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 __device__ __forceinline__ int64_t uniform64(int64_t v) {

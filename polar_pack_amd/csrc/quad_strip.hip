@@ -21,6 +21,7 @@
 // / 16.5 / 20.5 -> 10.7 / 11.7 / 13.9; N x K = 2048 x 11008 at 16 tokens 34.7 -> 27.2, 11008 x 2048
 // 46.0 -> 26.4.
 #include "rows_common.h"
+#include "slice_sums.h"
 
 #include <algorithm>
 
@@ -479,29 +480,6 @@ __global__ __launch_bounds__(QS_NT) void quad_strip_kernel(const QuadStripArgs A
   }
 }
 
-// out_m[j, n] = fp16(sum over slices of part), 4 columns a thread.
-__global__ __launch_bounds__(256) void quad_strip_finish_kernel(const QuadStripArgs A) {
-  const int64_t q4 = A.np / 4, total = 4ll * A.M * q4, at = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (at >= total) return;
-  const int64_t mj = at / q4;
-  const int n = (int)(at - mj * q4) * 4, m = (int)(mj / A.M), j = (int)(mj % A.M);
-  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 8
-  for (int s = 0; s < A.slices; ++s) {
-    const float4 p = *reinterpret_cast<const float4*>(A.part + ((int64_t)s * 4 * A.M + mj) * A.np + n);
-    v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
-  }
-  f16* o = model_out(A, m) + (int64_t)j * A.o_sm + (int64_t)n * A.o_sn;
-  if (A.vec_out && n + 3 < A.N) {
-    *reinterpret_cast<f16x4*>(o) = f16x4{(f16)v.x, (f16)v.y, (f16)v.z, (f16)v.w};
-  } else {
-    const float e[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      if (n + c < A.N) o[c * A.o_sn] = (f16)e[c];
-  }
-}
-
 // ------------------------------------------------------------------ host side
 struct StripPlan {
   int cols, strips, slices;
@@ -604,7 +582,17 @@ extern "C" int pp_quad_strip(const uint32_t* codes, int64_t ldk, const void* a, 
   else hipLaunchKernelGGL((quad_strip_kernel<2, 2>), grid, block, 0, st, A);
   PP_LAUNCH_CHECK();
   if (M > 1 && p.slices > 1) {
-    hipLaunchKernelGGL(quad_strip_finish_kernel, dim3((unsigned)((M * A.np + 255) / 256)), dim3(256), 0, st, A);
+    SliceSums<4> F = {};
+    F.part = A.part;
+    F.np = A.np;
+    for (int m = 0; m < 4; ++m) F.out[m] = A.out[m];
+    F.o_sm = o_sm;
+    F.o_sn = o_sn;
+    F.N = A.N;
+    F.M = A.M;
+    F.slices = A.slices;
+    F.vec_out = A.vec_out;
+    launch_slice_sums(F, st);
     PP_LAUNCH_CHECK();
   }
   return PP_OK;
