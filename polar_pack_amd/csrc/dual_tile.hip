@@ -12,10 +12,9 @@
 // 11008 x 2048 at 3 / 16 / 32 tokens 78.1 / 79.9 / 83.3 -> 34.3 / 35.5 / 36.2 us; 2048 x 11008 at 1 / 16
 // 58.0 / 59.3 -> 34.5 / 36.2; 4096 x 4096 at 16 46.5 -> 28.4; 1000 x 512 at 5 17.8 -> 11.7.
 #include "dual_lds.h"
+#include "row_tiles.h"
 #include "rows_common.h"
 #include "slice_sums.h"
-
-#include <algorithm>
 
 namespace pp {
 
@@ -23,11 +22,11 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-constexpr int DT_WAVES = 8, DT_NT = 64 * DT_WAVES;
-constexpr int64_t DT_MAX_M = 32, DT_MAX_GROUP = 8;
+constexpr int DT_NT = 64 * RT_WAVES;
+constexpr int64_t DT_MAX_M = 32;
 constexpr int DT_CAP = 960;                               // a wavefront's plug entries in LDS
 template <int T> constexpr int DT_SUB = T == 1 ? 4 : 2;   // steps a load stage
-static_assert(DLDS_BYTES + DT_WAVES * DT_CAP * 4 <= 160 * 1024, "tables and entries must fit a CU's LDS");
+static_assert(DLDS_BYTES + RT_WAVES * DT_CAP * 4 <= 160 * 1024, "tables and entries must fit a CU's LDS");
 
 struct DualTileArgs {
   const uint16_t* codes;   // row n at codes + n*ldc
@@ -50,16 +49,6 @@ struct DualTileArgs {
   int64_t plug_n;
   float* part;             // slices > 1: float32 sums, [slice][model][token][16 tiles]
 };
-
-// Columns [kb, ke) of a tile, a part of a wavefront's run.
-struct DtSeg {
-  int tile, kb, ke;
-};
-
-__device__ __forceinline__ void dt_run(int steps, int w, int& a, int& b) {
-  a = w * steps / DT_WAVES;
-  b = (w + 1) * steps / DT_WAVES;
-}
 
 // The chunk index and offset of a lane's next load position (no division but at a segment's start).
 struct DtPos {
@@ -88,7 +77,7 @@ struct DtStage {
 // have resources of no bytes; rows past N lie past the resource's end.  Neighbouring steps share the
 // codes' lines, so the loads keep the caches' policy.
 template <int T>
-__device__ __forceinline__ void dt_issue(const DualTileArgs& A, const DtSeg& S, int k, DtPos& pos, uint32_t voc,
+__device__ __forceinline__ void dt_issue(const DualTileArgs& A, const RowSeg& S, int k, DtPos& pos, uint32_t voc,
                                          const uint32_t (&vox)[T], DtStage<T>& D) {
   const int nrows = min(16, A.N - 16 * S.tile);
 #pragma unroll
@@ -114,7 +103,7 @@ struct DtPlugs {
   int n = 0, base = 0;     // lane l < 32: list l's entries and its first place in LDS
   bool held = true;        // the lists are in LDS
 
-  __device__ __forceinline__ void find(const DualTileArgs& A, const DtSeg (&S)[2], int lane) {
+  __device__ __forceinline__ void find(const DualTileArgs& A, const RowSeg (&S)[2], int lane) {
     const int64_t top = A.pos0 + (int64_t)min(A.N, 16 * (S[1].tile + 1)) * A.ldc;
     const int tile = lane >= 32 ? S[1].tile : S[0].tile, row = 16 * tile + (lane & 15);
     const int kb = lane >= 32 ? S[1].kb : S[0].kb, ke = lane >= 32 ? S[1].ke : S[0].ke;
@@ -145,7 +134,7 @@ struct DtPlugs {
     at = lo;
   }
   // The lists into the wave's part of LDS: (column from the segment's first) << 16 | amplitude.
-  __device__ __forceinline__ void keep(const DualTileArgs& A, const DtSeg (&S)[2], int lane, uint32_t* ent) {
+  __device__ __forceinline__ void keep(const DualTileArgs& A, const RowSeg (&S)[2], int lane, uint32_t* ent) {
     const int s = lane >> 4 & 1, row = 16 * (s ? S[1].tile : S[0].tile) + (lane & 15);
     const int b = __shfl(at, 32 * s + (lane & 15)), e = __shfl(at, 32 * s + 16 + (lane & 15));
     const bool some = s ? S[1].ke > S[1].kb : S[0].ke > S[0].kb;
@@ -169,7 +158,7 @@ struct DtPlugs {
 #pragma unroll
       for (int o = 16; o > 0; o >>= 1) l += __shfl(base, l + o) <= t ? o : 0;
       const int src = __shfl(b, l) + t - __shfl(base, l);
-      const DtSeg g = (l & 16) ? S[1] : S[0];
+      const RowSeg g = (l & 16) ? S[1] : S[0];
       const int64_t first = A.pos0 + (int64_t)(16 * g.tile + (l & 15)) * A.ldc + g.kb;
       const uint32_t k = A.plug_idx[from + src] - (uint32_t)first;
       const uint32_t amp = __builtin_bit_cast(unsigned short, A.plug_amp[from + src]);
@@ -181,7 +170,7 @@ struct DtPlugs {
 template <int T>
 struct DtRun {
   const DualTileArgs& A;
-  DtSeg S[2];
+  RowSeg S[2];
   int nseg;
   uint32_t voc, vox[T];
   int ri, q;
@@ -197,7 +186,7 @@ struct DtRun {
   __device__ __forceinline__ int64_t row_pos(int tile) const { return A.pos0 + (int64_t)(16 * tile + ri) * A.ldc; }
 
   // The next entry of the row in segment s.
-  __device__ __forceinline__ void entry(const DtSeg& s) {
+  __device__ __forceinline__ void entry(const RowSeg& s) {
     if (next >= end) {
       near = 0x7FFFFFFF;
     } else if (held) {
@@ -216,7 +205,7 @@ struct DtRun {
   __device__ __forceinline__ bool step(const char* lds, const DualLane& dl, const DtStage<T>& cur, DtStage<T>& pre,
                                        int& sg, int& k) {
     constexpr int SUB = DT_SUB<T>;
-    const DtSeg s = sg == 0 ? S[0] : S[1];
+    const RowSeg s = sg == 0 ? S[0] : S[1];
     int nsg = sg, nk = k + 32 * SUB;
     if (nk >= s.ke) {
       nsg = sg + 1;
@@ -311,21 +300,14 @@ __device__ __forceinline__ void dt_store(const DualTileArgs& A, int slice, int m
 
 template <int T, int LAYOUT>
 __global__ __launch_bounds__(DT_NT) void dual_tile_kernel(const DualTileArgs A) {
-  __shared__ __attribute__((aligned(16))) char lds[DLDS_BYTES + DT_WAVES * DT_CAP * 4];
-  static_assert(DT_WAVES * 2 * 2 * T * 64 * 16 <= DLDS_BYTES, "the runs' sums must fit where the tables were");
+  __shared__ __attribute__((aligned(16))) char lds[DLDS_BYTES + RT_WAVES * DT_CAP * 4];
+  static_assert(RT_WAVES * 2 * 2 * T * 64 * 16 <= DLDS_BYTES, "the runs' sums must fit where the tables were");
   const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6), ri = lane & 15, q = lane >> 4;
-  const int slice = blockIdx.x % A.slices, t0 = (int)(blockIdx.x / A.slices) * A.group;
-  const int ntiles = min(A.group, A.tiles - t0);
-  const int all = A.K / 32, s0 = (int)((int64_t)slice * all / A.slices), s1 = (int)((int64_t)(slice + 1) * all / A.slices);
-  const int per = s1 - s0, steps = ntiles * per;        // steps of a tile, of the workgroup
-  int a, b;
-  dt_run(steps, wave, a, b);
-  const int ta = a / per;
+  const RowShare W(A, wave);
   DtRun<T> R{A};
-  R.nseg = b <= a ? 0 : b > (ta + 1) * per ? 2 : 1;
-  R.S[0] = DtSeg{t0 + min(ta, ntiles - 1), 32 * (s0 + a - ta * per), 32 * (s0 + min(b - ta * per, per))};
-  R.S[1] = R.nseg == 2 ? DtSeg{t0 + ta + 1, 32 * s0, 32 * (s0 + b - (ta + 1) * per)}
-                       : DtSeg{R.S[0].tile, R.S[0].ke, R.S[0].ke};
+  R.nseg = W.nseg;
+  R.S[0] = W.S[0];
+  R.S[1] = W.S[1];
   R.ri = ri;
   R.q = q;
   R.voc = 2u * (uint32_t)(ri * A.ldc + 8 * q);
@@ -379,52 +361,15 @@ __global__ __launch_bounds__(DT_NT) void dual_tile_kernel(const DualTileArgs A) 
       if (!R.template step<LAYOUT>(lds, dl, D1, D0, sg, k)) break;
     }
   }
-  // the runs' sums, [wave][segment][model][token tile][lane], where the tables were
-  __syncthreads();
-  f4* red = reinterpret_cast<f4*>(lds);
-  auto slot = [&](int w, int sg, int m, int t) { return red + ((((w * 2 + sg) * 2 + m) * T + t) << 6) + lane; };
-#pragma unroll
-  for (int m = 0; m < 2; ++m)
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      if (R.nseg == 2) *slot(wave, 0, m, t) = R.H[m][t];
-      if (R.nseg > 0) *slot(wave, R.nseg - 1, m, t) = R.C[m][t];
-    }
-  __syncthreads();
-  for (int u = wave; u < ntiles * 2 * T; u += DT_WAVES) {
-    const int tile = u / (2 * T), m = u / T % 2, t = u % T;
-    f4 v = f4{0.f, 0.f, 0.f, 0.f};
-    for (int w = 0; w < DT_WAVES; ++w) {
-      int wa, wb;
-      dt_run(steps, w, wa, wb);
-      if (max(wa, tile * per) >= min(wb, (tile + 1) * per)) continue;
-      v += *slot(w, wa / per == tile ? 0 : 1, m, t);
-    }
-    dt_store(A, slice, m, 16 * t + ri, 16 * (t0 + tile) + 4 * q, v);
-  }
+  __syncthreads();         // every wave is done with the tables
+  row_sums<2, T>(reinterpret_cast<f4*>(lds), W, R, wave, lane, [&](int tile, int m, int t, f4 v) {
+    dt_store(A, W.slice, m, 16 * t + ri, 16 * (W.t0 + tile) + 4 * q, v);
+  });
 }
 
 // ------------------------------------------------------------------ host side
-struct DualTilePlan {
-  int group, slices;
-};
-
-// As quad_tile.hip's plan; a step takes about half as long, so a second pass counts 8 of them.
-static DualTilePlan dual_tile_plan(int64_t N, int64_t K) {
-  const int64_t cus = device_cu_count(), tiles = (N + 15) / 16, steps = K / 32;
-  DualTilePlan best = {};
-  int64_t least = INT64_MAX;
-  for (int64_t s = 1; s <= std::min<int64_t>({16, cus, std::max<int64_t>(1, steps / DT_WAVES)}); ++s) {
-    const int64_t groups = cus / s, group = (tiles + groups - 1) / groups, per = (steps + s - 1) / s;
-    if (group > DT_MAX_GROUP) break;
-    const int64_t cost = (group * per + DT_WAVES - 1) / DT_WAVES + (s > 1 ? 8 : 0);
-    if (cost < least) {
-      least = cost;
-      best = {(int)group, (int)s};
-    }
-  }
-  return best;
-}
+// A step takes about half as long as the quad kernel's, so a second pass counts 8 of them.
+static RowPlan dual_tile_plan(int64_t N, int64_t K) { return row_plan(N, K, 8); }
 
 }  // namespace pp
 
@@ -441,7 +386,7 @@ extern "C" int pp_dual_tile_ok(int64_t ldc, int64_t elem_base, int64_t a_sm, int
 
 extern "C" int64_t pp_dual_tile_workspace_size(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || N < 1 || K < 32) return 0;
-  const DualTilePlan p = dual_tile_plan(N, K);
+  const RowPlan p = dual_tile_plan(N, K);
   return p.slices > 1 ? (int64_t)p.slices * 2 * M * ((N + 15) / 16 * 16) * (int64_t)sizeof(float) : 0;
 }
 
@@ -460,7 +405,7 @@ extern "C" int pp_dual_tile(const void* codes, int code_layout, int64_t ldc, int
   PP_REQUIRE(n_groups >= 1 && n_groups < (1ll << 30), "n_groups must be in [1, 2^30)");
   PP_REQUIRE(o_sm >= N, "o_sm must be >= N");
   PP_REQUIRE(plug_n == 0 || (plug_idx && plug_amp), "plug arrays are null");
-  const DualTilePlan p = dual_tile_plan(N, K);
+  const RowPlan p = dual_tile_plan(N, K);
   const int64_t need = pp_dual_tile_workspace_size(M, N, K);
   PP_REQUIRE(need == 0 || (workspace != nullptr && workspace_bytes >= need && aligned(workspace, 16)),
              "workspace too small or misaligned: need %lld bytes", (long long)need);

@@ -15,16 +15,15 @@
 // Per call in a graph (0.1 % plug), against quad_mfma_kernel: 11008 x 2048 at 5 / 16 tokens 46.3 / 49.4
 // -> 30.8 / 31.9 us; 4096 x 4096 38.1 / 38.7 -> 24.1 / 24.6; 2048 x 2048 28.5 / 24.7 -> 14.6 / 15.4.
 #include "quad_mfma.h"
+#include "row_tiles.h"
 #include "slice_sums.h"
-
-#include <algorithm>
 
 namespace pp {
 
 typedef float f2 __attribute__((ext_vector_type(2)));
 
-constexpr int QT_WAVES = 8, QT_NT = 64 * QT_WAVES;
-constexpr int64_t QT_MAX_M = 32, QT_MAX_GROUP = 8;
+constexpr int QT_NT = 64 * RT_WAVES;
+constexpr int64_t QT_MAX_M = 32;
 // Steps a load stage (3 fit the registers beside two tiles' sums, and were 1 us slower at 16 tokens).
 template <int T> constexpr int QT_SUB = T == 1 ? 2 : 1;
 
@@ -45,17 +44,6 @@ struct QuadTileArgs {
   float* part;             // slices > 1: float32 sums, [slice][model][token][16 tiles]
 };
 
-// Columns [kb, ke) of a tile, a part of a wavefront's run.
-struct TileSeg {
-  int tile, kb, ke;
-};
-
-// Wave w's run [a, b) of the workgroup's steps.
-__device__ __forceinline__ void tile_run(int steps, int w, int& a, int& b) {
-  a = w * steps / QT_WAVES;
-  b = (w + 1) * steps / QT_WAVES;
-}
-
 template <int T>
 struct TileStage {
   u32x4 c[QT_SUB<T>][2];   // per step: 8 code words of the lane's row
@@ -67,7 +55,7 @@ struct TileStage {
 // loads share each 128-byte line, so the codes keep the caches' policy: with the streaming one
 // 11008 x 2048 at 16 tokens took 35.6 us for 32.3.
 template <int T>
-__device__ __forceinline__ void tile_issue(const QuadTileArgs& A, const TileSeg& S, int k, uint32_t voc,
+__device__ __forceinline__ void tile_issue(const QuadTileArgs& A, const RowSeg& S, int k, uint32_t voc,
                                            const uint32_t (&vox)[T], TileStage<T>& D) {
   const int nrows = min(16, A.N - 16 * S.tile);
 #pragma unroll
@@ -90,7 +78,7 @@ __device__ __forceinline__ void tile_issue(const QuadTileArgs& A, const TileSeg&
 struct TilePlugs {
   int64_t from = 0;
   int at = 0;              // lane 16 a + i: entry from + at
-  __device__ __forceinline__ void find(const QuadTileArgs& A, const TileSeg (&S)[2], int lane) {
+  __device__ __forceinline__ void find(const QuadTileArgs& A, const RowSeg (&S)[2], int lane) {
     const int64_t top = A.pos0 + (int64_t)min(A.N, 16 * (S[1].tile + 1)) * A.ldc;
     const int tile = lane >= 32 ? S[1].tile : S[0].tile, row = 16 * tile + (lane & 15);
     const int kb = lane >= 32 ? S[1].kb : S[0].kb, ke = lane >= 32 ? S[1].ke : S[0].ke;
@@ -118,7 +106,7 @@ struct TilePlugs {
     }
   }
   // The row's entries of segment s.
-  __device__ __forceinline__ void range(const QuadTileArgs& A, const TileSeg& S, int s, int ri, int64_t& next, int64_t& end) const {
+  __device__ __forceinline__ void range(const QuadTileArgs& A, const RowSeg& S, int s, int ri, int64_t& next, int64_t& end) const {
     const int b = __shfl(at, 32 * s + ri), e = __shfl(at, 32 * s + 16 + ri);
     const bool ok = 16 * S.tile + ri < A.N && S.ke > S.kb;
     next = ok ? from + b : 0;
@@ -203,7 +191,7 @@ __device__ __forceinline__ void tile_patch(const PlugSrc& S, MPlug& P, int& near
 template <int T>
 struct TileRun {
   const QuadTileArgs& A;
-  TileSeg S[2];
+  RowSeg S[2];
   int nseg;
   uint32_t voc, vox[T];
   int ri, q;
@@ -302,21 +290,14 @@ __device__ __forceinline__ void tile_store(const QuadTileArgs& A, int slice, int
 template <int T>
 __global__ __launch_bounds__(QT_NT) void quad_tile_kernel(const QuadTileArgs A) {
   __shared__ __attribute__((aligned(16))) uint32_t Tb[QLDS_BYTES / 4];
-  static_assert(QT_WAVES * 2 * 4 * T * 64 * 16 <= QLDS_BYTES, "the runs' sums must fit where the tables were");
+  static_assert(RT_WAVES * 2 * 4 * T * 64 * 16 <= QLDS_BYTES, "the runs' sums must fit where the tables were");
   char* lds = reinterpret_cast<char*>(Tb);
   const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6), ri = lane & 15, q = lane >> 4;
-  const int slice = blockIdx.x % A.slices, t0 = (int)(blockIdx.x / A.slices) * A.group;
-  const int ntiles = min(A.group, A.tiles - t0);
-  const int all = A.K / 32, s0 = (int)((int64_t)slice * all / A.slices), s1 = (int)((int64_t)(slice + 1) * all / A.slices);
-  const int per = s1 - s0, steps = ntiles * per;        // steps of a tile, of the workgroup
-  int a, b;
-  tile_run(steps, wave, a, b);
-  const int ta = a / per;
+  const RowShare W(A, wave);
   TileRun<T> R{A};
-  R.nseg = b <= a ? 0 : b > (ta + 1) * per ? 2 : 1;
-  R.S[0] = TileSeg{t0 + min(ta, ntiles - 1), 32 * (s0 + a - ta * per), 32 * (s0 + min(b - ta * per, per))};
-  R.S[1] = R.nseg == 2 ? TileSeg{t0 + ta + 1, 32 * s0, 32 * (s0 + b - (ta + 1) * per)}
-                       : TileSeg{R.S[0].tile, R.S[0].ke, R.S[0].ke};
+  R.nseg = W.nseg;
+  R.S[0] = W.S[0];
+  R.S[1] = W.S[1];
   R.ri = ri;
   R.q = q;
   R.voc = 4u * (uint32_t)(ri * A.ldc + 8 * q);
@@ -354,54 +335,15 @@ __global__ __launch_bounds__(QT_NT) void quad_tile_kernel(const QuadTileArgs A) 
   }
   if (shared) R.template walk<LayShared>(lds, LayShared::lane(lane), D);
   else R.template walk<LaySplit>(lds, LaySplit::lane(lane), D);
-  // the runs' sums, [wave][segment][model][token tile][lane], where the tables were
-  __syncthreads();
-  f4* red = reinterpret_cast<f4*>(lds);
-  auto slot = [&](int w, int sg, int m, int t) { return red + ((((w * 2 + sg) * 4 + m) * T + t) << 6) + lane; };
-#pragma unroll
-  for (int m = 0; m < 4; ++m)
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      if (R.nseg == 2) *slot(wave, 0, m, t) = R.H[m][t];
-      if (R.nseg > 0) *slot(wave, R.nseg - 1, m, t) = R.C[m][t];
-    }
-  __syncthreads();
-  for (int u = wave; u < ntiles * 4 * T; u += QT_WAVES) {
-    const int tile = u / (4 * T), m = u / T % 4, t = u % T;
-    f4 v = f4{0.f, 0.f, 0.f, 0.f};
-    for (int w = 0; w < QT_WAVES; ++w) {
-      int wa, wb;
-      tile_run(steps, w, wa, wb);
-      if (max(wa, tile * per) >= min(wb, (tile + 1) * per)) continue;
-      v += *slot(w, wa / per == tile ? 0 : 1, m, t);
-    }
-    tile_store(A, slice, m, 16 * t + ri, 16 * (t0 + tile) + 4 * q, v);
-  }
+  __syncthreads();         // every wave is done with the tables
+  row_sums<4, T>(reinterpret_cast<f4*>(lds), W, R, wave, lane, [&](int tile, int m, int t, f4 v) {
+    tile_store(A, W.slice, m, 16 * t + ri, 16 * (W.t0 + tile) + 4 * q, v);
+  });
 }
 
 // ------------------------------------------------------------------ host side
-struct TilePlan {
-  int group, slices;
-};
-
-// Slices of K and tiles a workgroup, one round of workgroups on the chip: the least of the
-// longest wave's steps, with 5 for a second pass over the slices' sums (a step of 8 wavefronts
-// takes about 1 us, the pass 4-5).  No plan (group 0) past 8 tiles a workgroup.
-static TilePlan tile_plan(int64_t N, int64_t K) {
-  const int64_t cus = device_cu_count(), tiles = (N + 15) / 16, steps = K / 32;
-  TilePlan best = {};
-  int64_t least = INT64_MAX;
-  for (int64_t s = 1; s <= std::min<int64_t>({16, cus, std::max<int64_t>(1, steps / QT_WAVES)}); ++s) {
-    const int64_t groups = cus / s, group = (tiles + groups - 1) / groups, per = (steps + s - 1) / s;
-    if (group > QT_MAX_GROUP) break;
-    const int64_t cost = (group * per + QT_WAVES - 1) / QT_WAVES + (s > 1 ? 5 : 0);
-    if (cost < least) {
-      least = cost;
-      best = {(int)group, (int)s};
-    }
-  }
-  return best;
-}
+// A step of 8 wavefronts takes about 1 us, a second pass 4-5.
+static RowPlan tile_plan(int64_t N, int64_t K) { return row_plan(N, K, 5); }
 
 }  // namespace pp
 
@@ -415,7 +357,7 @@ extern "C" int pp_quad_tile_ok(int64_t ldc, int64_t a_sm, int64_t plug_n, int64_
 
 extern "C" int64_t pp_quad_tile_workspace_size(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || N < 1 || K < 32) return 0;
-  const TilePlan p = tile_plan(N, K);
+  const RowPlan p = tile_plan(N, K);
   return p.slices > 1 ? (int64_t)p.slices * 4 * M * ((N + 15) / 16 * 16) * (int64_t)sizeof(float) : 0;
 }
 
@@ -432,7 +374,7 @@ extern "C" int pp_quad_tile(const uint32_t* codes, int64_t ldc, int64_t elem_bas
              "operands the tile kernel does not read");
   PP_REQUIRE(o_sm >= N, "o_sm must be >= N");
   PP_REQUIRE(plug_n == 0 || (plug_idx && plug_vals), "plug arrays are null");
-  const TilePlan p = tile_plan(N, K);
+  const RowPlan p = tile_plan(N, K);
   const int64_t need = pp_quad_tile_workspace_size(M, N, K);
   PP_REQUIRE(need == 0 || (workspace != nullptr && workspace_bytes >= need && aligned(workspace, 16)),
              "workspace too small or misaligned: need %lld bytes", (long long)need);
