@@ -363,3 +363,21 @@ def test_quad_split_tables_every_route(layout, M):
     for k in range(4):
         ref[k][at] = vals[:, k].astype(np.float64) * scales[k]
         assert_dequant_close(w[k].cpu().numpy(), ref[k], f"dequant model {k}")
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("N,K", [(1, 4), (1, 1024), (9, 256), (64, 1028), (300, 516), (2049, 512), (17_000, 64)])
+def test_rows_with_idle_waves(N, K, M):
+    """(N,K) rows on the one-Linear launch with workgroups and waves that have no task (their first
+    loads hold no bytes), one chunk and more a wave, whole rows and column slices, with plug entries."""
+    rng = np.random.default_rng(N + K + M)
+    codes = random_codes((N, K), N + K)
+    luts, scales = fp16_luts(N + M)
+    flat = np.sort(rng.choice(N * K, max(1, N * K // 50), replace=False)).astype(np.uint32)
+    vals = (rng.standard_normal((flat.size, 4)) * 0.5).astype(np.float16)
+    a = rng.standard_normal((M, K)).astype(np.float16)
+    view = u32(codes).to(DEV).t()
+    assert qk.quad_call_route(view, M, flat.size) == "rows"
+    outs = qk.quad_bitpacked(torch.from_numpy(a).to(DEV), view, [l.to(DEV) for l in luts], scales,
+                             plug=(u32(flat + np.uint32(7)).to(DEV), torch.from_numpy(vals).to(DEV)), elem_base=7)
+    check_route(outs, a, np.ascontiguousarray(codes.T), luts, scales, "fused", (flat % K, flat // K), vals, f"{N}x{K}")
