@@ -131,6 +131,10 @@ struct QuadTableBuild {
     for (int i = 0; i < 4; ++i) v[i] = lut_val<E>(luts, 1 + i, e);
     U.template load<E>(luts);
   }
+  // Waits for every LUT load.
+  __device__ __forceinline__ void wait() const {
+    asm volatile("" : : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(U.r), "v"(U.c1), "v"(U.s1), "v"(U.c3), "v"(U.s3));
+  }
   // Whether this thread's q1 and q2 entries agree (waits for the first LUT loads only).
   __device__ __forceinline__ bool same() const {
     return __float_as_uint(v[0]) == __float_as_uint(v[2]) && __float_as_uint(v[1]) == __float_as_uint(v[3]);

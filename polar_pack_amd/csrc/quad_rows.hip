@@ -710,7 +710,10 @@ __device__ __forceinline__ void rows_body(const char* lds, const QuadRowsArgs& A
 // where after a second barrier the slice-0 wave adds them and writes the outputs.
 // ONE: every wave has at most one task (SegRunner::run_one): its first two chunks and its
 // plug positions are requested before the build.
-template <int MT, typename E, int PARTS, bool ONE>
+// ALL: a wave without a task issues the first chunk's loads too, with no bytes, and all wait for the LUT
+// values before the second.  Under a branch the compiler's waits for those values count on the path
+// without the chunks, so they cover the chunks in flight (see direct_all).
+template <int MT, typename E, int PARTS, bool ONE, bool ALL>
 __device__ __forceinline__ void direct_body(uint32_t* T, const QuadRowsArgs& A, int64_t gw) {
   constexpr int RG = RowsCfg<MT>::RG, NSEG = RowsCfg<MT>::NSEG, NT = RowsCfg<MT>::NT, WAVES = NT / 64;
   constexpr bool SPLIT = PARTS != 0, WG = PARTS == 2;
@@ -746,24 +749,20 @@ __device__ __forceinline__ void direct_body(uint32_t* T, const QuadRowsArgs& A, 
 #pragma unroll
   for (int r = 0; r < RG; ++r) voff[r] = 4u * (uint32_t)(r * S.ldc) + 16u * lane;
   Chunk<MT, RG, NSEG> c0, c1;
-  // 1 us faster than after the build.  A wave without a task issues the same loads, with no bytes: were
-  // they under a branch, the compiler's waits below would count on the shorter path and cover the chunks
-  // in flight before the tables (1531 x 4104 at 1 token 11.5 us, 10.7 this way; 2048 x 2048 8.2, 7.5).
-  const int kb = busy ? S.kbeg : 0;
-  chunk_issue<MT, RG, NSEG>(S, 0, kb, voff, lane, c0, busy);
+  if (ALL || busy) chunk_issue<MT, RG, NSEG>(S, 0, busy ? S.kbeg : 0, voff, lane, c0, busy);   // 1 us faster than after the build
   // the caller's plan, kept inside the table whatever it holds (a stale plan must not send
   // the plug loads outside it)
   const int64_t pc = std::min<int64_t>(std::max<int64_t>(uniform64((int64_t)(((uint64_t)wp[1] << 32) | wp[0])), 0),
                                        A.plug_n);
   uint32_t idx0 = 0;
-  if (ONE) vload32(idx0, 4u * lane, plug_idx_rsrc(A, busy ? pc : A.plug_n));
+  if (ALL) tb.wait();
   const bool same = tb.same();
-  if (ONE) {
-    // the second chunk once the first LUT values are back (issued with the first, gate
+  if (ONE && busy) {
+    // the second chunk once the LUT values are back (issued with the first, gate
     // 11008x2048 built its tables 4.9 us after entry; 4.7 this way, both 25.1-26.2 us)
-    const int k1 = kb + NSEG * QSEG;
-    const bool more = busy && k1 < S.kend;
-    chunk_issue<MT, RG, NSEG>(S, 0, more ? k1 : kb, voff, lane, c1, more);
+    vload32(idx0, 4u * lane, plug_idx_rsrc(A, pc));
+    const int k1 = S.kbeg + NSEG * QSEG;
+    chunk_issue<MT, RG, NSEG>(S, 0, k1 < S.kend ? k1 : S.kbeg, voff, lane, c1, k1 < S.kend);
   }
   const bool shared = tb.finish(T, A.luts, same);
   if (!WG && !busy) return;
@@ -811,12 +810,12 @@ __global__ __launch_bounds__(RowsCfg<MT>::NT) void quad_rows_kernel(const QuadRo
 
 // One Linear (segs == nullptr): a kernel of its own, so that the whole-stream kernel keeps
 // its register allocation.  PARTS as direct_body.
-template <int MT, int PARTS, bool ONE = false>
+template <int MT, int PARTS, bool ONE, bool ALL>
 __global__ __launch_bounds__(RowsCfg<MT>::NT) void quad_direct_kernel(const QuadRowsArgs A) {
   __shared__ __attribute__((aligned(16))) uint32_t T[QLDS_BYTES / 4];
   const int64_t gw = (int64_t)blockIdx.x * (RowsCfg<MT>::NT / 64) + uniform(threadIdx.x >> 6);
-  if (A.luts.dtype == PP_F16) direct_body<MT, f16, PARTS, ONE>(T, A, gw);
-  else direct_body<MT, float, PARTS, ONE>(T, A, gw);
+  if (A.luts.dtype == PP_F16) direct_body<MT, f16, PARTS, ONE, ALL>(T, A, gw);
+  else direct_body<MT, float, PARTS, ONE, ALL>(T, A, gw);
 }
 
 // ------------------------------------------------------------------ tail rows
@@ -957,7 +956,14 @@ static int cfg_waves(int mt) {
   }
 }
 
-template <int PARTS>
+// Whether every wave issues the first chunk's loads (direct_body's ALL): from 2 M code words.  Below,
+// the chunks are back as soon as the LUT values and the idle waves' empty loads only cost time.  Per call
+// in a graph, with the branch / without, at 1, 2 and 4 tokens: 128 x 64 5.6 / 5.7, 5.5 / 5.7, 5.4 / 5.7
+// us; 1440 x 1216 7.6 / 7.8, 8.1 / 8.3, 9.0 / 8.8; 500 x 4100 11.1 / 10.4, 8.7 / 8.2, 10.0 / 9.4; 2048 x
+// 2048 8.7 / 8.1, 9.8 / 9.7, 10.9 / 10.6; 4096 x 4096 18.8 / 17.8, 19.5 / 18.2, 24.6 / 24.2.
+static bool direct_all(const QuadRowsArgs& A) { return (int64_t)A.proj.N * A.proj.K >= 1 << 21; }
+
+template <int PARTS, bool ALL>
 static void launch_direct_t(const QuadRowsArgs& A, int mt, hipStream_t st) {
   const unsigned grid = (unsigned)device_cu_count();
   // at most one task per wave: a task per column slice per wave at most (direct_item deals
@@ -966,21 +972,27 @@ static void launch_direct_t(const QuadRowsArgs& A, int mt, hipStream_t st) {
   const bool one = PARTS == 2 || A.n_tasks <= W / std::max(1, A.parts);
   switch (mt) {
     case 1:
-      if (one) hipLaunchKernelGGL((quad_direct_kernel<1, PARTS, true>), dim3(grid), dim3(RowsCfg<1>::NT), 0, st, A);
-      else hipLaunchKernelGGL((quad_direct_kernel<1, PARTS>), dim3(grid), dim3(RowsCfg<1>::NT), 0, st, A);
+      if (one) hipLaunchKernelGGL((quad_direct_kernel<1, PARTS, true, ALL>), dim3(grid), dim3(RowsCfg<1>::NT), 0, st, A);
+      else hipLaunchKernelGGL((quad_direct_kernel<1, PARTS, false, ALL>), dim3(grid), dim3(RowsCfg<1>::NT), 0, st, A);
       break;
-    case 2: hipLaunchKernelGGL((quad_direct_kernel<2, PARTS>), dim3(grid), dim3(RowsCfg<2>::NT), 0, st, A); break;
-    case 4: hipLaunchKernelGGL((quad_direct_kernel<4, PARTS>), dim3(grid), dim3(RowsCfg<4>::NT), 0, st, A); break;
-    default: hipLaunchKernelGGL((quad_direct_kernel<8, PARTS>), dim3(grid), dim3(RowsCfg<8>::NT), 0, st, A); break;
+    case 2: hipLaunchKernelGGL((quad_direct_kernel<2, PARTS, false, ALL>), dim3(grid), dim3(RowsCfg<2>::NT), 0, st, A); break;
+    case 4: hipLaunchKernelGGL((quad_direct_kernel<4, PARTS, false, ALL>), dim3(grid), dim3(RowsCfg<4>::NT), 0, st, A); break;
+    default: hipLaunchKernelGGL((quad_direct_kernel<8, PARTS, false, ALL>), dim3(grid), dim3(RowsCfg<8>::NT), 0, st, A); break;
   }
+}
+
+template <int PARTS>
+static void launch_direct(const QuadRowsArgs& A, int mt, hipStream_t st) {
+  if (direct_all(A)) launch_direct_t<PARTS, true>(A, mt, st);
+  else launch_direct_t<PARTS, false>(A, mt, st);
 }
 
 template <bool SPLIT>
 static void launch_rows_t(const QuadRowsArgs& A, int mt, hipStream_t st) {
   const unsigned grid = (unsigned)device_cu_count();
   if (A.segs == nullptr) {
-    if (SPLIT && A.wg_parts) launch_direct_t<2>(A, mt, st);
-    else launch_direct_t<SPLIT ? 1 : 0>(A, mt, st);
+    if (SPLIT && A.wg_parts) launch_direct<2>(A, mt, st);
+    else launch_direct<SPLIT ? 1 : 0>(A, mt, st);
     return;
   }
   switch (mt) {

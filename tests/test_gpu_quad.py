@@ -366,7 +366,8 @@ def test_quad_split_tables_every_route(layout, M):
 
 
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
-@pytest.mark.parametrize("N,K", [(1, 4), (1, 1024), (9, 256), (64, 1028), (300, 516), (2049, 512), (17_000, 64)])
+@pytest.mark.parametrize("N,K", [(1, 4), (1, 1024), (9, 256), (64, 1028), (300, 516), (2049, 512), (17_000, 64), (1200, 1764),
+                                 (33_000, 64), (520, 4100)])
 def test_rows_with_idle_waves(N, K, M):
     """(N,K) rows on the one-Linear launch with workgroups and waves that have no task (their first
     loads hold no bytes), one chunk and more a wave, whole rows and column slices, with plug entries."""
