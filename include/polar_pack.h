@@ -372,7 +372,8 @@ int pp_plug_search(const uint32_t* plug_idx, int64_t plug_n, int64_t pos0, int64
  *   pp_quad_strip_ok              1 if it reads these operands: lut_dtype PP_F16, K % 8 == 0 (M > 1:
  *                                 K % 32 == 0), N and ldk multiples of 4 words and codes 16-byte
  *                                 aligned to 16 tokens (2 words, 8 bytes above), activations
- *                                 16-byte aligned with a_sm % 8 == 0, K * ldk < 2^29
+ *                                 16-byte aligned with a_sm % 8 == 0, K * ldk < 2^29, and at one
+ *                                 token K * N < 26,214,400 (above, pp_quad_gemm is the faster one)
  *   pp_quad_strip_workspace_size  bytes of workspace (the slices' float32 sums; any contents)
  *   pp_quad_strip_counts          bytes of counts, zero on entry and left zero (one token in several
  *                                 slices; launches that share them must not overlap)

@@ -33,6 +33,11 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int QS_WAVES = 8, QS_NT = 64 * QS_WAVES;
 constexpr int64_t QS_MAX_M = 32;
+// Code words to which one token takes the strips: above, quad_kn_kernel reads the codes faster (a
+// wavefront 1 KiB of a row at a time, where a strip takes 256 bytes).  Strips / row kernel at K x N of 13 M
+// words 19.4 / 22.4 us, 24 M 28.0 / 28.4, 25 M 25.7-27.7 / 27.3-27.8, 28 M 34.3 / 31.9, 45 M 41.5 / 40.0,
+// 67 M 59.1 / 53.0, 89 M 82.9 / 72.5.
+constexpr int64_t QS_GEMV_WORDS = 25ll << 20;
 
 struct QuadStripArgs {
   const uint32_t* codes;   // code of (row 0, column 0); row k at codes + k*ldk
@@ -517,7 +522,7 @@ extern "C" int pp_quad_strip_ok(const void* codes, int64_t ldk, const void* a, i
                                 int64_t N, int64_t K) {
   if (lut_dtype != PP_F16 || M < 1 || M > QS_MAX_M || N < 1 || K < 32 || ldk < N) return 0;
   if (K * ldk >= (1ll << 29) || !aligned(a, 16) || (M > 1 && (a_sm < K || a_sm % 8 != 0))) return 0;
-  if (M * (M > 1 ? a_sm : K) >= (1ll << 29)) return 0;
+  if (M * (M > 1 ? a_sm : K) >= (1ll << 29) || (M == 1 && K * N >= QS_GEMV_WORDS)) return 0;
   // 16-byte code loads to 16 tokens, 8-byte ones above
   const int unit = M <= 16 ? 4 : 2;
   return K % (M == 1 ? 8 : 32) == 0 && N % unit == 0 && ldk % unit == 0 && aligned(codes, 4 * unit);

@@ -100,6 +100,24 @@ def test_several_slices_and_rounds(M, K, N):
     check([g[:, torch.from_numpy(cols).to(DEV)] for g in first], exact, f"M={M}")
 
 
+@pytest.mark.parametrize("K,N,strip", [(4096, 6396, True), (4096, 6400, False), (8192, 8192, False)])
+def test_one_token_of_a_large_layer(K, N, strip):
+    """From 25 Mi words on one token takes the row kernel, which is the faster one there; other tokens
+    and the outputs do not depend on it (float32 weights and sums either way)."""
+    ok = nat.lib().pp_quad_strip_ok
+    assert bool(ok(0, N, 0, K, nat.PP_F16, 1, N, K)) == strip and ok(0, N, 0, K, nat.PP_F16, 16, N, K)
+    if N > 6400:
+        return
+    g = torch.Generator(device=DEV).manual_seed(N)
+    words = torch.randint(-2 ** 31, 2 ** 31 - 1, (K, N), generator=g, device=DEV, dtype=torch.int64).int()
+    luts, scales = fp16_luts(N)
+    a = np.random.default_rng(N).standard_normal((1, K)).astype(np.float16)
+    got = qk.quad_bitpacked(torch.from_numpy(a).to(DEV), words.view(torch.uint32), [t.to(DEV) for t in luts], scales)
+    exact = kn_mfma_reference(a, words[:, ::101].cpu().numpy().view(np.uint32), luts, scales)[0]
+    for m in range(4):
+        assert_gemv_close(got[m][:, ::101].float().cpu().numpy(), exact[m], f"model {m}", rtol=5.1e-4)
+
+
 @pytest.mark.parametrize("M", [1, 2, 16, 17, 32])
 @pytest.mark.parametrize("K,N", [(256, 72), (2080, 1000)])
 def test_float32_tables_keep_the_other_kernels(K, N, M):
