@@ -10,8 +10,8 @@
 // atomic adds and launches to find the rows' plug entries and to read the sums back.  Here a
 // wavefront finds its rows' entries itself while the LUTs travel, and one slice needs no second
 // launch.  The decode takes ~19 vector instructions and 4 LDS reads (14 LDS clocks a wavefront) a
-// word; at two wavefronts a SIMD, all the tables leave room for, the vector units are busy 41 % and
-// LDS 21 % of the time (SQ counters), so what bounds it is the latency of a step's loads and lookups.
+// word; at two wavefronts a SIMD, all the tables leave room for, the vector units are busy 45 % and
+// LDS 23 % of the time (SQ counters), so what bounds it is the latency of a step's loads and lookups.
 // Per call in a graph (0.1 % plug), against quad_mfma_kernel: 11008 x 2048 at 5 / 16 tokens 46.3 / 49.4
 // -> 30.8 / 31.9 us; 4096 x 4096 38.1 / 38.7 -> 24.1 / 24.6; 2048 x 2048 28.5 / 24.7 -> 14.6 / 15.4.
 #include "quad_mfma.h"
