@@ -223,16 +223,14 @@ def packable(ws) -> bool:
                 or torch.autograd.forward_ad._current_level >= 0)
 
 
-def upload(hosts, dev):
-    """Device copies of small contiguous host tensors (each a multiple of 4 bytes), every one with
-    storage of its own, carried in the launches' arguments (pp_upload): unlike ``host.to(dev)`` it
-    does not wait for queued work."""
-    import torch
-    outs = [torch.empty(h.shape, dtype=h.dtype, device=dev) for h in hosts]
-    sizes = (i64 * len(hosts))(*[h.numel() * h.element_size() for h in hosts])
-    check(lib().pp_upload(ptr_array([o.data_ptr() for o in outs]), ptr_array([h.data_ptr() for h in hosts]), sizes,
-                          len(hosts), raw_stream(dev)), "pp_upload")
-    return outs
+def upload(outs, sources):
+    """Small host arrays (at the addresses ``sources``) into the device tensors ``outs``, of a multiple
+    of 4 bytes each, carried in the launches' arguments (pp_upload): unlike a copy from pageable memory
+    it does not wait for queued work.  The host memory may change once the call returns."""
+    n = len(outs)
+    sizes = (i64 * n)(*[o.numel() * o.element_size() for o in outs])
+    check(lib().pp_upload(ptr_array([o.data_ptr() for o in outs]), ptr_array(sources), sizes, n,
+                          raw_stream(outs[0].device)), "pp_upload")
 
 
 def plug_search(idx, n: int, pos0: int, pld: int, rows: int, slices: int, cols: int, dev):

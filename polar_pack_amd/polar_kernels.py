@@ -24,6 +24,7 @@ torch.matmul).
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import torch
@@ -68,16 +69,27 @@ def quantize_polar_bitpacked(w1, w2, amp_bits=6, num_phases=1024, mu=255, group_
     amp_q = torch.round(compressed * levels).clamp(0, levels).to(torch.int8).flatten()[:total].reshape(K, N)
     bmax = bmax.flatten().to(torch.float16)
     packed = pack_amp_phase(amp_q, phase_q)
-    amp_lut, cos_lut, sin_lut = (t.to(w1.device) for t in _layer_luts(levels, num_phases, mu, log_mu))
+    amp_lut, cos_lut, sin_lut = (t.to(w1.device) for t in _layer_luts(mu, log_mu, _lut_arguments(levels, num_phases)))
     return packed, bmax, amp_lut, cos_lut, sin_lut
 
 
-def _layer_luts(levels, num_phases, mu, log_mu):
-    """(amp_lut, cos_lut, sin_lut) of a packed layer as fp16 host tensors (polar_kernels.py:142-150);
-    they depend on nothing but the code's parameters."""
-    phases = torch.linspace(-math.pi, math.pi, num_phases + 1)[:-1]
-    i = torch.arange(levels + 1, dtype=torch.float32)
-    return (((torch.exp(i / levels * log_mu) - 1.0) / mu).to(torch.float16), torch.cos(phases).to(torch.float16),
+def _lut_arguments(levels, num_phases):
+    """What the LUTs' functions are taken of: i / levels and the phase codes' angles."""
+    return (torch.arange(levels + 1, dtype=torch.float32) / levels,
+            torch.linspace(-math.pi, math.pi, num_phases + 1)[:-1])
+
+
+@functools.lru_cache(maxsize=8)
+def _host_lut_arguments(levels, num_phases, default_dtype):
+    """:func:`_lut_arguments` on the host (linspace follows torch's default dtype, hence the key)."""
+    return _lut_arguments(levels, num_phases)
+
+
+def _layer_luts(mu, log_mu, arguments):
+    """(amp_lut, cos_lut, sin_lut) of a packed layer as fp16 tensors (polar_kernels.py:142-150); they
+    depend on nothing but the code's parameters."""
+    u, phases = arguments
+    return (((torch.exp(u * log_mu) - 1.0) / mu).to(torch.float16), torch.cos(phases).to(torch.float16),
             torch.sin(phases).to(torch.float16))
 
 
@@ -103,8 +115,10 @@ def _pack_dual_device(w1, w2, levels, num_phases, mu, log_mu, group_size):
                                          num_phases, levels, mu, log_mu, packed.data_ptr(), bmax.data_ptr(),
                                          nat.raw_stream(dev)), "pp_dual_pack")
         # the host's work while the pass runs
-        amp_lut, cos_lut, sin_lut = nat.upload(_layer_luts(levels, num_phases, mu, log_mu), dev)
-    return packed, bmax, amp_lut, cos_lut, sin_lut
+        host = _layer_luts(mu, log_mu, _host_lut_arguments(levels, num_phases, torch.get_default_dtype()))
+        luts = [torch.empty(t.shape, dtype=torch.float16, device=dev) for t in host]
+        nat.upload(luts, [t.data_ptr() for t in host])
+    return packed, bmax, *luts
 
 
 def _lut_dtype(*ts):

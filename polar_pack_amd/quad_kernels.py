@@ -26,6 +26,7 @@ from __future__ import annotations
 
 import collections
 import ctypes
+import functools
 import math
 import threading
 import weakref
@@ -68,19 +69,27 @@ def pack_quad_layer(w1, w2, w3, w4, mu=MU):
     q2 = torch.round(t2 / math.pi * 255).clip(0, 255)
     q3 = torch.round(t3 / (2 * math.pi) * 255).clip(0, 255)
     codes = _u32_words(nq, q1, q2, q3)
-    growth, angles = _lut_tables(mu)
-    luts = [t.to(torch.float16).to(w1.device) for t in (growth * r_max / mu, *angles)]
+    growth, cos, sin = _lut_tables(mu, _lut_arguments())
+    luts = [(growth * r_max / mu).to(torch.float16), *(t[turn].clone() for turn in (0, 0, 1) for t in (cos, sin))]
+    luts = [t.to(w1.device) for t in luts]
     return codes, luts, [float(sk) for sk in s]
 
 
-def _lut_tables(mu):
-    """What a layer's LUTs hold whatever its weights, in float32: exp(i/255 ln(1+mu)) - 1, which
-    r_max / mu scales to the norms, and the six angle tables (quad_kernels.py:39-49)."""
+def _lut_arguments():
+    """What the LUTs' functions are taken of: i/255, and the half and the full turn in its steps."""
     u = torch.arange(256, dtype=torch.float32) / 255
-    half_turn = u * math.pi
-    full_turn = u * 2 * math.pi
-    cos, sin = torch.cos(half_turn), torch.sin(half_turn)
-    return torch.exp(u * math.log1p(mu)) - 1, (cos, sin, cos, sin, torch.cos(full_turn), torch.sin(full_turn))
+    return u, torch.stack([u * math.pi, u * 2 * math.pi])
+
+
+_host_lut_arguments = functools.lru_cache(maxsize=1)(_lut_arguments)
+
+
+def _lut_tables(mu, arguments):
+    """What a layer's LUTs hold whatever its weights (quad_kernels.py:39-49): exp(i/255 ln(1+mu)) - 1 in
+    float32, which r_max / mu scales to the norms, and the cosines and sines of the half and the full
+    turn as the rows of two fp16 tensors."""
+    u, turns = arguments
+    return torch.exp(u * math.log1p(mu)) - 1, torch.cos(turns).to(torch.float16), torch.sin(turns).to(torch.float16)
 
 
 def _pack_quad_device(ws, mu):
@@ -110,12 +119,14 @@ def _pack_quad_device(ws, mu):
         known.record()
         nat.check(L.pp_quad_pack_codes(ptrs, dtype, n, mu, log_mu, meta.data_ptr(), codes.data_ptr(), stream),
                   "pp_quad_pack_codes")
-        # the host's work while the device's passes run (the two polar angles share their tables)
-        growth, (cos, sin, _, _, *turn) = _lut_tables(mu)
-        cos, sin, *turn = (t.to(torch.float16) for t in (cos, sin, *turn))
+        # the host's work while the device's passes run
+        growth, cos, sin = _lut_tables(mu, _host_lut_arguments())
+        luts = [torch.empty(256, dtype=torch.float16, device=dev) for _ in range(7)]
         known.synchronize()
         *scales, top = host.tolist()
-        luts = nat.upload([(growth * (top * 1.001) / mu).to(torch.float16), cos, sin, cos, sin, *turn], dev)
+        norms = (growth * (top * 1.001) / mu).to(torch.float16)
+        c, s = cos.data_ptr(), sin.data_ptr()           # the two polar angles' tables are the same
+        nat.upload(luts, [norms.data_ptr(), c, s, c, s, c + 512, s + 512])
     return codes.view(torch.uint32), luts, scales
 
 
