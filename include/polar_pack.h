@@ -369,11 +369,13 @@ int pp_plug_search(const uint32_t* plug_idx, int64_t plug_n, int64_t pos0, int64
 /*
  * Fused decode of (K,N) codes (unit column stride, row stride ldk words) with fp16 tables for 1
  * to 32 tokens, no plug table (quad_kernels.py:103-159): strips of columns x slices of K.
- *   pp_quad_strip_ok              1 if it reads these operands: lut_dtype PP_F16, K % 8 == 0 (M > 1:
+ *   pp_quad_strip_ok              1 if it reads these operands and is the kernel for them: lut_dtype
+ *                                 PP_F16, K % 8 == 0 (M > 1:
  *                                 K % 32 == 0), N and ldk multiples of 4 words and codes 16-byte
  *                                 aligned to 16 tokens (2 words, 8 bytes above), activations
- *                                 16-byte aligned with a_sm % 8 == 0, K * ldk < 2^29, and at one
- *                                 token K * N < 26,214,400 (above, pp_quad_gemm is the faster one)
+ *                                 16-byte aligned with a_sm % 8 == 0, K * ldk < 2^29; at one token
+ *                                 K * N < 26,214,400 (pp_quad_strip takes more, pp_quad_gemm is
+ *                                 the faster one there)
  *   pp_quad_strip_workspace_size  bytes of workspace (the slices' float32 sums; any contents)
  *   pp_quad_strip_counts          bytes of counts, zero on entry and left zero (one token in several
  *                                 slices; launches that share them must not overlap)
@@ -455,11 +457,13 @@ int pp_quad_pack_codes(const void* const* w, int dtype, int64_t n, double mu, do
                        uint32_t* codes, void* stream);
 
 /*
- * count tables, bytes[t] (a multiple of 4) of host memory at src[t] to device memory at dst[t], in the
- * launches' own arguments (3,584 bytes a launch): the host memory is read before the call returns and
- * nothing waits for earlier work.  For tables of a few KB.  No counterpart in the reference.
+ * pp_upload: bytes (a multiple of 4) of host memory to the device in the launches' own arguments
+ * (3,584 bytes a launch): the host memory is read before the call returns and nothing waits for
+ * earlier work.  pp_upload_tables: count of them, bytes[t] from src[t] to dst[t], sharing launches.
+ * For tables of a few KB.  No counterpart in the reference.
  */
-int pp_upload(void* const* dst, const void* const* src, const int64_t* bytes, int count, void* stream);
+int pp_upload(void* dst, const void* src, int64_t bytes, void* stream);
+int pp_upload_tables(void* const* dst, const void* const* src, const int64_t* bytes, int count, void* stream);
 
 /* ------------------------------------------------------------------------ */
 /* Dual pack: 16-bit [amp 6 | phase 10] -> 2 models.                          */

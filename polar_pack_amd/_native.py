@@ -133,7 +133,8 @@ EXPORTS = {
     "pp_quad_pack_norm": (i32, [vp, i32, i64, vp, vp, vp]),
     "pp_quad_pack_codes": (i32, [vp, i32, i64, f64, f64, vp, vp, vp]),
     "pp_dual_pack": (i32, [vp, vp, i32, i64, i64, i64, i32, f64, f64, vp, vp, vp]),
-    "pp_upload": (i32, [vp, vp, vp, i32, vp]),
+    "pp_upload": (i32, [vp, vp, i64, vp]),
+    "pp_upload_tables": (i32, [vp, vp, vp, i32, vp]),
 }
 
 _lock = threading.Lock()
@@ -225,12 +226,12 @@ def packable(ws) -> bool:
 
 def upload(outs, sources):
     """Small host arrays (at the addresses ``sources``) into the device tensors ``outs``, of a multiple
-    of 4 bytes each, carried in the launches' arguments (pp_upload): unlike a copy from pageable memory
-    it does not wait for queued work.  The host memory may change once the call returns."""
+    of 4 bytes each, carried in the launches' arguments (pp_upload_tables): unlike a copy from
+    pageable memory it does not wait for queued work.  The host memory may change once the call returns."""
     n = len(outs)
     sizes = (i64 * n)(*[o.numel() * o.element_size() for o in outs])
-    check(lib().pp_upload(ptr_array([o.data_ptr() for o in outs]), ptr_array(sources), sizes, n,
-                          raw_stream(outs[0].device)), "pp_upload")
+    check(lib().pp_upload_tables(ptr_array([o.data_ptr() for o in outs]), ptr_array(sources), sizes, n,
+                                 raw_stream(outs[0].device)), "pp_upload_tables")
 
 
 def plug_search(idx, n: int, pos0: int, pld: int, rows: int, slices: int, cols: int, dev):

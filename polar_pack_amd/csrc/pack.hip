@@ -347,7 +347,8 @@ extern "C" int pp_dual_pack(const void* w1, const void* w2, int dtype, int64_t n
   return PP_OK;
 }
 
-extern "C" int pp_upload(void* const* dst, const void* const* src, const int64_t* bytes, int count, void* stream) {
+extern "C" int pp_upload_tables(void* const* dst, const void* const* src, const int64_t* bytes, int count,
+                                void* stream) {
   PP_REQUIRE(count >= 0 && (count == 0 || (dst && src && bytes)), "null pointer argument");
   for (int t = 0; t < count; ++t) {
     PP_REQUIRE(bytes[t] >= 0 && bytes[t] % 4 == 0, "bytes must be a multiple of 4");
@@ -382,4 +383,8 @@ extern "C" int pp_upload(void* const* dst, const void* const* src, const int64_t
     PP_LAUNCH_CHECK();
   }
   return PP_OK;
+}
+
+extern "C" int pp_upload(void* dst, const void* src, int64_t bytes, void* stream) {
+  return pp_upload_tables(&dst, &src, &bytes, 1, stream);
 }

@@ -514,18 +514,23 @@ static StripPlan strip_plan(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
+static bool strip_reads(const void* codes, int64_t ldk, const void* a, int64_t a_sm, int lut_dtype, int64_t M, int64_t N,
+                        int64_t K) {
+  if (lut_dtype != PP_F16 || M < 1 || M > QS_MAX_M || N < 1 || K < 32 || ldk < N) return false;
+  if (K * ldk >= (1ll << 29) || !aligned(a, 16) || (M > 1 && (a_sm < K || a_sm % 8 != 0))) return false;
+  if (M * (M > 1 ? a_sm : K) >= (1ll << 29)) return false;
+  // 16-byte code loads to 16 tokens, 8-byte ones above
+  const int unit = M <= 16 ? 4 : 2;
+  return K % (M == 1 ? 8 : 32) == 0 && N % unit == 0 && ldk % unit == 0 && aligned(codes, 4 * unit);
+}
+
 }  // namespace pp
 
 using namespace pp;
 
 extern "C" int pp_quad_strip_ok(const void* codes, int64_t ldk, const void* a, int64_t a_sm, int lut_dtype, int64_t M,
                                 int64_t N, int64_t K) {
-  if (lut_dtype != PP_F16 || M < 1 || M > QS_MAX_M || N < 1 || K < 32 || ldk < N) return 0;
-  if (K * ldk >= (1ll << 29) || !aligned(a, 16) || (M > 1 && (a_sm < K || a_sm % 8 != 0))) return 0;
-  if (M * (M > 1 ? a_sm : K) >= (1ll << 29) || (M == 1 && K * N >= QS_GEMV_WORDS)) return 0;
-  // 16-byte code loads to 16 tokens, 8-byte ones above
-  const int unit = M <= 16 ? 4 : 2;
-  return K % (M == 1 ? 8 : 32) == 0 && N % unit == 0 && ldk % unit == 0 && aligned(codes, 4 * unit);
+  return strip_reads(codes, ldk, a, a_sm, lut_dtype, M, N, K) && (M > 1 || K * N < QS_GEMV_WORDS);
 }
 
 extern "C" int64_t pp_quad_strip_counts(int64_t M, int64_t N, int64_t K) {
@@ -546,7 +551,7 @@ extern "C" int pp_quad_strip(const uint32_t* codes, int64_t ldk, const void* a, 
                              int64_t counts_bytes, void* stream) {
   PP_REQUIRE(codes != nullptr && a != nullptr && out != nullptr && luts != nullptr && scales != nullptr,
              "null pointer argument");
-  PP_REQUIRE(pp_quad_strip_ok(codes, ldk, a, a_sm, lut_dtype, M, N, K), "operands the strip kernel does not read");
+  PP_REQUIRE(strip_reads(codes, ldk, a, a_sm, lut_dtype, M, N, K), "operands the strip kernel does not read");
   for (int m = 0; m < 4; ++m) PP_REQUIRE(out[m] != nullptr, "out[%d] is null", m);
   for (int i = 0; i < 7; ++i) PP_REQUIRE(luts[i] != nullptr, "lut %d is null", i);
   const StripPlan p = strip_plan(M, N, K);

@@ -17,12 +17,14 @@ Quad kernels (the reference's one fused kernel, quad_kernels.py:53-159, at every
 
 * ``rows``     fused row decode of (N,K) rows seen as (K,N) (the container stream layout),
                1-8 tokens (``pp_quad_gemm`` -> ``quad_rows_kernel``)
-* ``kn``       fused row decode of (K,N) codes with unit column stride (``pack_quad_layer``),
-               8 tokens per pass (``pp_quad_gemm`` -> ``quad_kn_kernel``)
+* ``kn``       fused row decode of (K,N) codes with unit column stride (``pack_quad_layer``): one token
+               without plug entries, fp16 tables, below 25 Mi words ``pp_quad_strip``, else 8 tokens
+               per pass (``pp_quad_gemm`` -> ``quad_kn_kernel``)
 * ``mfma``     matrix-core batch decode of (N,K) rows, 1-64 tokens per launch (``pp_quad_tile`` to
                32 tokens, else ``pp_quad_mfma``)
 * ``big_nk``   fused matrix-core kernel on (N,K) rows, blocks of 16-256 tokens (``pp_quad_big``)
-* ``big_kn``   the same kernel on (K,N) codes as stored
+* ``big_kn``   the same kernel on (K,N) codes as stored (``pp_quad_strip`` to 32 tokens without plug
+               entries, fp16 tables)
 * ``kn_mfma``  (K,N) codes transposed into (N,K) rows, then ``mfma`` (``fused=False`` only)
 * ``prefill``  fp16 decode + one batched library GEMM (hipBLASLt through ``torch.matmul``)
 * ``generic``  any strides: decode into a float32 workspace, then a plain GEMV kernel

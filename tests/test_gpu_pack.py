@@ -173,5 +173,7 @@ def test_upload_of_several_tables(sizes):
     hosts = [torch.randint(-2 ** 31, 2 ** 31 - 1, (n,), generator=g, dtype=torch.int32) for n in sizes]
     outs = [torch.empty(n, dtype=torch.int32, device=DEV) for n in sizes]
     nat.upload(outs, [h.data_ptr() for h in hosts])
-    for got, want in zip(outs, hosts):
+    one = torch.zeros_like(outs[0])
+    nat.check(nat.lib().pp_upload(one.data_ptr(), hosts[0].data_ptr(), 4 * sizes[0], nat.raw_stream(DEV)), "pp_upload")
+    for got, want in zip([*outs, one], [*hosts, hosts[0]]):
         assert torch.equal(got.cpu(), want)
